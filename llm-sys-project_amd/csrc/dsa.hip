@@ -107,12 +107,17 @@ constexpr int kT32 = 32;
 constexpr int kStage32 = kT32 * kRowBytes;                // 36864
 constexpr int kMaxSplitS = 65536;                         // selected positions per query (32 splits)
 constexpr int kTileBlocks = kStage32 / 1024;              // 36 DMA instructions per tile
+constexpr int kTrans = 4;                                 // positions per thread and round of the translation
 template <int NW> struct SplitGeom {                      // NW waves
     static constexpr int RING = NW == 8 ? 4 : 3;
     static constexpr int CHUNK = NW == 8 ? 2048 : kMaxS;  // most tokens per split
+    static constexpr int ROUND = kTrans * 64 * NW;        // positions the workgroup translates per round
     static constexpr int ROWS = RING * kStage32;          // LDS offsets: the tokens' cache rows,
-    static constexpr int MASK = ROWS + CHUNK * 4;         // their validity bits, 64 per word
-    static constexpr int LDS = MASK + CHUNK / 8;
+    static constexpr int MASK = ROWS + CHUNK * 4;         // their validity bits, 64 per word:
+    // a round writes all of its words, past the split too (6 waves: 3 rounds
+    // of 1536 positions for 4096)
+    static constexpr int LDS = MASK + (CHUNK + ROUND - 1) / ROUND * (ROUND / 8);
+    static_assert(LDS <= 160 * 1024 && MASK % 8 == 0, "split kernel LDS");
 };
 
 __device__ __forceinline__ int tile32_off(int t, int j) {  // token t (0..31), chunk j (0..71)
@@ -173,7 +178,7 @@ __device__ __forceinline__ void dsa_split_body(
     // page), its page id is >= 0 and its row inside the cache; an invalid
     // one (e.g. the -1 padding of a sequence shorter than the selection)
     // reads no page-table entry, loads a zero row and scores -inf.
-    constexpr int kPer = 4;  // split positions per thread and round
+    constexpr int kPer = kTrans;
     const int* lg = logical + (size_t)qi * S + t0;
     const int* pt = page_table + (size_t)qi * pages_per_seq;
     const long seq = (long)pages_per_seq * page;
@@ -206,7 +211,7 @@ __device__ __forceinline__ void dsa_split_body(
     };
     // (8 waves take a split's 2048 positions in one round)
     if constexpr (NW < 8)
-        for (int r0 = kPer * kThreads; r0 < len; r0 += kPer * kThreads) lookup(r0), to_rows(r0);
+        for (int r0 = G::ROUND; r0 < len; r0 += G::ROUND) lookup(r0), to_rows(r0);
     lookup(0);
     __builtin_amdgcn_sched_barrier(0);
     // q of head hbase + c16 as B fragments: K-step ks = 32 dims, group g holds 8
@@ -700,7 +705,10 @@ int launch_dsa_bf16_paged(const uint16_t* qn, const uint16_t* qp, const uint16_t
                  : hg == 96 ? dsa_split96_kernel
                  : hg == 64 ? (wide ? dsa_split64_wide_kernel : dsa_split64_kernel)
                             : (wide ? dsa_split32_wide_kernel : dsa_split32_kernel);
-    const int lds = hg == 128 ? SplitGeom<8>::LDS : SplitGeom<4>::LDS;
+    const int lds = hg == 128  ? SplitGeom<8>::LDS
+                    : hg == 96 ? SplitGeom<6>::LDS
+                    : hg == 64 ? SplitGeom<4>::LDS
+                               : SplitGeom<2>::LDS;
     const int rc = ensure_dynamic_lds((const void*)split, lds);
     if (rc != AMDMOE_OK) return rc;
     hipLaunchKernelGGL(split, dim3((unsigned)grid), dim3(4 * hg), lds, st, qn, qp, cache,

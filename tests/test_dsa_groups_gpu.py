@@ -30,6 +30,7 @@ SHAPES = [
     (70, 96, 600, 1024),  # 96-head groups
     (300, 32, 64, 256),   # more groups than CUs, one split each
     (130, 64, 2050, 4096),  # one split of more than 2048 positions
+    (130, 96, 3072, 4096), (130, 96, 3073, 4096), (131, 96, 4096, 4096),  # 96-head groups: rounds of 1536 positions
     (1, 128, 2048, 4096), (3, 256, 65, 256), (64, 128, 64, 256), (1, 384, 4096, 8192),  # H a multiple of 128
     (1, 128, 4097, 8192),  # past the small groups' positions: 128 heads
 ]
