@@ -73,8 +73,12 @@ typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
 // ring (each tile's loads go out two tiles ahead), filled by direct
 // global->LDS loads; each wave reads every tile once for S and once for V.
 // dsa_split96/64/32_kernel are the same body with 6, 4 and 2 waves, for groups
-// of that many heads where H is no multiple of 128: no skew between waves, so
-// a 3-stage ring and room for the rows of 4096 positions.
+// of that many heads: no skew between waves, so a 3-stage ring and room for the
+// rows of 4096 positions.  A wave alone on its SIMD waits for LDS and for its
+// own softmax (1.5 us per tile for 0.45 of MFMAs), and with 32 heads half of
+// the SIMDs have none: dsa_split32x2_kernel gives every second tile to a second
+// pair of waves and adds the two sums up in LDS at the end.  One split of 32 heads
+// over 2048 positions: 103.9 -> 59.5 us (Q=1), 216 -> 186 (Q=300).
 //   S^T (16 tokens x 16 heads) = K . Q^T   16x16x32 bf16, 2 token tiles,
 //                                          q of the wave's 16 heads in
 //                                          registers
@@ -108,11 +112,11 @@ constexpr int kStage32 = kT32 * kRowBytes;                // 36864
 constexpr int kMaxSplitS = 65536;                         // selected positions per query (32 splits)
 constexpr int kTileBlocks = kStage32 / 1024;              // 36 DMA instructions per tile
 constexpr int kTrans = 4;                                 // positions per thread and round of the translation
-template <int NW> struct SplitGeom {                      // NW waves
-    static constexpr int RING = NW == 8 ? 4 : 3;
-    static constexpr int CHUNK = NW == 8 ? 2048 : kMaxS;  // most tokens per split
-    static constexpr int ROUND = kTrans * 64 * NW;        // positions the workgroup translates per round
-    static constexpr int ROWS = RING * kStage32;          // LDS offsets: the tokens' cache rows,
+template <int NH, int TG> struct SplitGeom {              // TG groups of NH waves
+    static constexpr int RING = NH == 8 ? 4 : (TG > 1 ? 2 : 3);  // stages per group
+    static constexpr int CHUNK = NH == 8 ? 2048 : (TG > 1 ? 3072 : kMaxS);  // most tokens per split
+    static constexpr int ROUND = kTrans * 64 * NH * TG;   // positions the workgroup translates per round
+    static constexpr int ROWS = TG * RING * kStage32;     // LDS offsets: the tokens' cache rows,
     static constexpr int MASK = ROWS + CHUNK * 4;         // their validity bits, 64 per word:
     // a round writes all of its words, past the split too (6 waves: 3 rounds
     // of 1536 positions for 4096)
@@ -139,21 +143,24 @@ static __device__ __align__(16) uint16_t g_dsa_zero_row[kDt];
 // the output rows; otherwise it writes its partial, (max, sum) per head and
 // the unnormalised O: bf16 for 128-head groups (the merge adds at most a few
 // in fp32), fp32 for the smaller ones.
-template <bool WIDE, int NW>
+template <bool WIDE, int NH, int TG>
 __device__ __forceinline__ void dsa_split_body(
     const uint16_t* __restrict__ qn, const uint16_t* __restrict__ qp,
     const uint16_t* __restrict__ cache, long cache_bytes, const int* __restrict__ page_table,
     const int* __restrict__ logical, uint16_t* __restrict__ out, void* __restrict__ part,
     float* __restrict__ part_ml, int Q, int H, int S, int page, int pages_per_seq, int nsplit, int chunk,
     float scale_log2) {
-    using G = SplitGeom<NW>;
-    constexpr int kHeads = 16 * NW, kThreads = 64 * NW, kRing32 = G::RING;
-    constexpr int kBlocks = kTileBlocks / NW;  // DMA instructions per wave and tile (8 waves: 4 or 5)
+    using G = SplitGeom<NH, TG>;
+    constexpr int NW = NH * TG, kHeads = 16 * NH, kThreads = 64 * NW, kRing32 = G::RING;
+    constexpr int kAhead = kRing32 > 2 ? 2 : 1;  // tiles loaded ahead
+    constexpr int kBlocks = kTileBlocks / NH;    // DMA instructions per wave and tile (8 waves: 4 or 5)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     int* s_rows = (int*)(smem + G::ROWS);
     unsigned long long* s_mask = (unsigned long long*)(smem + G::MASK);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hw = TG > 1 ? wave % NH : wave, tg = TG > 1 ? wave / NH : 0;  // heads and token group
+    uint8_t* const ring = smem + tg * kRing32 * kStage32;
     // work item lin = (query, head group, split), dealt to the 8 XCDs in
     // contiguous chunks (workgroup b runs on XCD b % 8): the splits of a
     // query share an XCD, so its q rows come from HBM once and its partials
@@ -168,7 +175,7 @@ __device__ __forceinline__ void dsa_split_body(
     const int t0 = sp * chunk;
     const int len = max(0, min(S, t0 + chunk) - t0);
     const int g = lane >> 4, c16 = lane & 15;
-    const int hbase = kHeads * hg + 16 * wave;  // this wave's first head
+    const int hbase = kHeads * hg + 16 * hw;  // this wave's first head
 
     // Prologue, ordered so the q loads overlap the two dependent loads of
     // the page-table translation: logical indices, then page-table entries,
@@ -210,7 +217,7 @@ __device__ __forceinline__ void dsa_split_body(
         }
     };
     // (8 waves take a split's 2048 positions in one round)
-    if constexpr (NW < 8)
+    if constexpr (NH < 8)
         for (int r0 = G::ROUND; r0 < len; r0 += G::ROUND) lookup(r0), to_rows(r0);
     lookup(0);
     __builtin_amdgcn_sched_barrier(0);
@@ -256,19 +263,19 @@ __device__ __forceinline__ void dsa_split_body(
             return vo;
         }
     };
-    // a tile's 36 blocks: wave w issues b = w + NW n (8 waves: n < 5 for waves
-    // 0-3 and n < 4 for waves 4-7)
+    // a tile's 36 blocks: wave w of its group issues b = w + NH n (8 waves: n < 5
+    // for waves 0-3 and n < 4 for waves 4-7)
     auto issue_blk = [&](int st, RowAddr vo0, RowAddr vo1, int n) __attribute__((always_inline)) {
-        const int b = wave + NW * n;
+        const int b = hw + NH * n;
         const int tg = b >= 18 ? 1 : 0;
         if constexpr (WIDE)
             __builtin_amdgcn_global_load_lds((gptr_t)((tg ? vo1 : vo0) + 64 * (b - 18 * tg)),
-                                             (lds_ptr_t)(smem + st * kStage32 + b * 1024), 16, 0, 0);
+                                             (lds_ptr_t)(ring + st * kStage32 + b * 1024), 16, 0, 0);
         else
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rc, (lds_ptr_t)(smem + st * kStage32 + b * 1024), 16, tg ? vo1 : vo0, 64 * (b - 18 * tg), 0, 0);
+                rc, (lds_ptr_t)(ring + st * kStage32 + b * 1024), 16, tg ? vo1 : vo0, 64 * (b - 18 * tg), 0, 0);
     };
-    const bool extra = kTileBlocks % NW != 0 && wave < kTileBlocks % NW;  // uniform: a fifth block per tile
+    const bool extra = kTileBlocks % NH != 0 && hw < kTileBlocks % NH;  // uniform: a fifth block per tile
     auto issue_tile = [&](int st, RowAddr vo0, RowAddr vo1) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < kBlocks; n++) issue_blk(st, vo0, vo1, n);
@@ -296,13 +303,17 @@ __device__ __forceinline__ void dsa_split_body(
     // after barrier n into the stage of tile n-2 (read until barrier n), and
     // every wave waits for its blocks of tile n before barrier n.  Each wave
     // passes ntiles + 1 barriers.
-    // With 4 or 2 waves there is one per SIMD and no lag: tile n is read
-    // between barriers n and n+1, and tile n+2 goes into the stage of n-1.
-    const bool lag = NW == 8 && wave >= 4;  // uniform
-    // prologue: tiles 0 and 1 (tiles past the end read zeros into their stage)
+    // The smaller groups have no lag: tile n is read between barriers n and
+    // n+1, and tile n+2 goes into the stage of n-1.  Two token groups have a
+    // ring of 2 stages each, for every second tile: tile n is their tile n/2, and
+    // the next one goes into the stage of the one before.
+    const bool lag = NH == 8 && wave >= 4;  // uniform
+    // prologue: the first tiles (tiles past the end read zeros into their stage)
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-        issue_tile(i, row_vo(kT32 * i + (lane >> 2)), row_vo(kT32 * i + 16 + (lane >> 2)));
+    for (int i = 0; i < kAhead; i++) {
+        const int tok = kT32 * (TG * i + tg) + (lane >> 2);
+        issue_tile(i, row_vo(tok), row_vo(tok + 16));
+    }
     // this wave's blocks of the older of its two tiles in flight have landed
     auto wait_older = [&]() __attribute__((always_inline)) {
         if (extra) wait_vmcnt<kBlocks + 1>();
@@ -315,7 +326,7 @@ __device__ __forceinline__ void dsa_split_body(
     auto s_phase = [&](auto issuec, uint32_t soff, int stn, RowAddr nvo0, RowAddr nvo1,
                        f32x4 (&sacc)[2]) __attribute__((always_inline)) {
         constexpr bool ISSUE = decltype(issuec)::value;
-        const uint8_t* kb = smem + soff;
+        const uint8_t* kb = ring + soff;
         constexpr int kPre = NW > 4 ? 2 : 6;  // (at most 4 waves: one per SIMD, with its registers)
         u32x4 a[18][2];
 #pragma unroll
@@ -382,7 +393,7 @@ __device__ __forceinline__ void dsa_split_body(
     auto pv_phase = [&](auto issuec, uint32_t soff, int stn, RowAddr nvo0, RowAddr nvo1,
                         const u32x4& pb) __attribute__((always_inline)) {
         constexpr bool ISSUE = decltype(issuec)::value;
-        const uint8_t* kb = smem + soff;
+        const uint8_t* kb = ring + soff;
         auto vfrag = [&](int mt) __attribute__((always_inline)) {
             const uint8_t* p = kb + vlo[mt & 1] + 1024 * (mt >> 1);
             const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)p);
@@ -416,18 +427,22 @@ __device__ __forceinline__ void dsa_split_body(
         // the q loads (older than the tile DMA) have landed: without this the
         // compiler waits for every load in flight, tile 1's included
         wait_older();
-        for (int t = 0; t < ntiles; t++) {
-            const int tn = t + 2;
-            const RowAddr nvo0 = row_vo(kT32 * tn + (lane >> 2)), nvo1 = row_vo(kT32 * tn + 16 + (lane >> 2));
-            wait_older();    // tile t landed (this wave's part); tile t+1 may stay in flight
-            bare_barrier();  // barrier t
-            const uint32_t soff = stage_of(t);
-            f32x4 sacc[2];
-            s_phase(on{}, soff, tn % kRing32, nvo0, nvo1, sacc);
-            const u32x4 pb = softmax(t, sacc);
-            pv_phase(off{}, soff, 0, nvo0, nvo1, pb);
+        for (int u = 0; u * TG < ntiles; u++) {  // uniform
+            const int t = TG * u + tg, un = u + kAhead;
+            const int tok = kT32 * (TG * un + tg) + (lane >> 2);
+            const RowAddr nvo0 = row_vo(tok), nvo1 = row_vo(tok + 16);
+            if constexpr (kAhead == 2) wait_older();  // tile t landed (this wave's part); tile t+1 may stay in flight
+            else wait_vmcnt<0>();
+            bare_barrier();  // barrier u
+            if (TG == 1 || t < ntiles) {  // uniform in the wave
+                const uint32_t soff = stage_of(u);
+                f32x4 sacc[2];
+                s_phase(on{}, soff, un % kRing32, nvo0, nvo1, sacc);
+                const u32x4 pb = softmax(t, sacc);
+                pv_phase(off{}, soff, 0, nvo0, nvo1, pb);
+            }
         }
-        if constexpr (NW == 8) bare_barrier();  // barrier ntiles
+        if constexpr (NH == 8) bare_barrier();  // barrier ntiles
     } else {
         wait_older();
         bare_barrier();  // barrier 0
@@ -446,8 +461,27 @@ __device__ __forceinline__ void dsa_split_body(
     }
     wait_vmcnt<0>();  // the trailing (out-of-range) tile loads
 
-    const float l = xor32_sum(xor16_sum(l_lane));
-    if (NW < 8 && nsplit == 1) {  // all of the query's positions: the output rows
+    float l = xor32_sum(xor16_sum(l_lane));
+    if constexpr (TG == 2) {  // the groups' sums, weighted as in the merge kernels
+        lds_barrier();        // every wave is past its last tile
+        float* xo = (float*)smem + hw * (64 * 130) + lane;  // 128 sums, max and sum per lane, 64 lanes apart
+        if (tg == 1) {
+#pragma unroll
+            for (int i = 0; i < 128; i++) xo[64 * i] = o[i >> 2][i & 3];
+            xo[64 * 128] = m_run;
+            xo[64 * 129] = l;
+        }
+        lds_barrier();
+        if (tg == 1) return;
+        const float m1 = xo[64 * 128], l1 = xo[64 * 129];
+        const float m = fmaxf(m_run, m1), mu = m == -INFINITY ? 0.0f : m;  // no valid position: weights 0
+        const float w0 = exp2f(m_run - mu), w1 = exp2f(m1 - mu);
+#pragma unroll
+        for (int i = 0; i < 128; i++) o[i >> 2][i & 3] = o[i >> 2][i & 3] * w0 + xo[64 * i] * w1;
+        l = l * w0 + l1 * w1;
+        m_run = m;
+    }
+    if (NH < 8 && nsplit == 1) {  // all of the query's positions: the output rows
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         uint16_t* orow = out + ((size_t)qi * H + hbase + c16) * kDc + 4 * g;
 #pragma unroll
@@ -459,7 +493,7 @@ __device__ __forceinline__ void dsa_split_body(
     // the split's partial in the accumulator order (each store contiguous
     // over the wave) and (max, sum) per head
     const size_t prow0 = ((size_t)qi * nsplit + sp) * H + hbase;
-    if constexpr (NW == 8) {
+    if constexpr (NH == 8) {
         uint16_t* pb_base = (uint16_t*)part + prow0 * kDc + (size_t)lane * 4;
 #pragma unroll
         for (int mt = 0; mt < 32; mt++)
@@ -473,23 +507,25 @@ __device__ __forceinline__ void dsa_split_body(
     if (g == 0) *(float2*)(part_ml + 2 * (prow0 + c16)) = make_float2(m_run, l);
 }
 
-#define AMDMOE_DSA_SPLIT_KERNEL(NAME, W, NW)                                                          \
-    __global__ __launch_bounds__(64 * NW, 1) void NAME(                                               \
+#define AMDMOE_DSA_SPLIT_KERNEL(NAME, W, NH, TG)                                                      \
+    __global__ __launch_bounds__(64 * NH * TG, 1) void NAME(                                          \
         const uint16_t* __restrict__ qn, const uint16_t* __restrict__ qp,                             \
         const uint16_t* __restrict__ cache, long cache_bytes, const int* __restrict__ page_table,     \
         const int* __restrict__ logical, uint16_t* __restrict__ out, void* __restrict__ part,         \
         float* __restrict__ part_ml, int Q, int H, int S, int page, int pages_per_seq, int nsplit,    \
         int chunk, float scale_log2) {                                                                \
-        dsa_split_body<W, NW>(qn, qp, cache, cache_bytes, page_table, logical, out, part, part_ml, Q, \
-                              H, S, page, pages_per_seq, nsplit, chunk, scale_log2);                  \
+        dsa_split_body<W, NH, TG>(qn, qp, cache, cache_bytes, page_table, logical, out, part,         \
+                                  part_ml, Q, H, S, page, pages_per_seq, nsplit, chunk, scale_log2);  \
     }
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split_kernel, false, 8)
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split_wide_kernel, true, 8)
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split96_kernel, false, 6)
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split64_kernel, false, 4)
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split32_kernel, false, 2)
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split64_wide_kernel, true, 4)
-AMDMOE_DSA_SPLIT_KERNEL(dsa_split32_wide_kernel, true, 2)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split_kernel, false, 8, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split_wide_kernel, true, 8, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split96_kernel, false, 6, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split64_kernel, false, 4, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split32_kernel, false, 2, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split32x2_kernel, false, 2, 2)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split64_wide_kernel, true, 4, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split32_wide_kernel, true, 2, 1)
+AMDMOE_DSA_SPLIT_KERNEL(dsa_split32x2_wide_kernel, true, 2, 2)
 #undef AMDMOE_DSA_SPLIT_KERNEL
 
 // Combines the splits of dsa_split_kernel: per (query, head), m = max of
@@ -624,46 +660,55 @@ __global__ __launch_bounds__(64) void dsa_merge_f32_kernel(const float* __restri
                                            pack_bf16x2(acc[k][2] * inv, acc[k][3] * inv)};
 }
 
+// us of a workgroup over n tiles; load: the share of the CUs that are busy.
+// Measured at Q = 1 .. 300, H = 32 .. 256, S = 64 .. 2048, every split count:
+// the first tile (page table, q) and a slope, which rises where the
+// workgroups share the memory (32 heads, S=2048 Q=1: 59.5, S=600 on 256 CUs: 28.5).
+static float split_us(int hg, int n, float load) {
+    if (hg == 32 && n > 2 && n * kT32 <= SplitGeom<2, 2>::CHUNK) return 8.8f + (0.8f + 0.24f * load) * n;
+    if (hg == 32) return 7.0f + (n > 2 ? 1.5f : 1.2f) * n;
+    if (hg == 64) return 8.3f + 1.58f * n;
+    if (hg == 96) return 11.0f + 1.5f * n;
+    return 8.4f + (1.8f + 0.5f * load) * n;
+}
+
 // Heads per workgroup, splits per query and the bytes of the splits'
 // partials.  Head groups of 128 (H a multiple of 128): enough workgroups to
 // cover the chip (256 CUs), at most 2048 tokens per split, at least 32.  Small
 // groups of 32, 64 or 96 heads (S <= 4096): any split that fits the CUs at
 // once, more than one only with stream scratch.  The cheapest by a model
-// fitted to measured calls (us; H = 32 .. 128, Q = 1 .. 300, S = 64 ..
-// 2048): a workgroup of 32 / 64 / 96 / 128 heads takes 7.0 /
-// 8.3 / 10.7 / 9.0 before its first tile (page table, q) and 1.2 / 1.4 / 1.5 /
-// 2.1 per tile of 32 tokens, workgroups run in rounds of 256, a merge takes 4
-// + 0.1 per split (0.5 in the 128-head merge, four splits a round trip) and
-// moves the partials at 8 MB per us.  So few queries take many splits of
-// small groups (S=2000 Q=4 H=64: 79 us in one split of 32 heads, 21 so; S=2048
-// Q=1 H=128: 48 us in 64 splits of 128 heads, 18 so), short selections one
-// split of small groups (S=64 Q=64 H=128: 20 -> 11), large batches 128 heads.
+// fitted to measured calls (us): workgroups run in rounds of 256, a merge takes
+// 4 + 0.2 per split (0.5 in the 128-head merge, four splits a round trip) and
+// moves its partials at 8 MB per us (16 where they are bf16).
+// So few queries take many splits of small groups (S=2000 Q=4 H=64: 61 us in one
+// split of 32 heads, 19 in 16; S=2048 Q=1 H=128: 48 us in 64 splits of 128 heads,
+// 17 so), short selections one split of small groups (S=64 Q=64 H=128: 20 ->
+// 10; S=512 Q=64 H=96: 24, 31 in 3 splits of 96), large batches 128 heads.
 DsaPlan dsa_paged_plan(int Q, int H, int S, bool scratch) {
     DsaPlan best = {0, 1, 0};
     if (Q < 1 || H < 32 || H % 32 != 0 || S < 1) return best;
     const int tiles = (S + kT32 - 1) / kT32;
     float best_us = 0.0f;
+    auto estimate = [&](int hg, int ns) {
+        const long wgs = (long)Q * (H / hg) * ns;
+        const float rounds = (float)((wgs + 255) / 256), load = std::min(1.0f, wgs / 256.0f);
+        float us = rounds * split_us(hg, (tiles + ns - 1) / ns, load);
+        if (hg == 128) us += 4.0f + 0.5f * ns + 2.0f * ns * Q * H * (kDc * 2) / 16e6f;
+        else if (ns > 1) us += 4.0f + 0.2f * ns + 2.0f * ns * Q * H * (kDc * 4) / 8e6f;
+        return us;
+    };
     if (H % 128 == 0) {
         const long wg = (long)Q * (H / 128);
         const int fill = (int)std::min<long>((256 + wg - 1) / wg, tiles);
-        const int ns = std::max(fill, (S + SplitGeom<8>::CHUNK - 1) / SplitGeom<8>::CHUNK);
-        const float rounds = (float)((wg * ns + 255) / 256);
-        best = {128, ns, 0};
-        // (a fifth less: the small groups' estimates run low where their
-        // workgroups share rows, e.g. 28.5 us measured for 26.2 at Q=32 S=512)
-        best_us = 0.8f * (rounds * (9.0f + 2.1f * ((tiles + ns - 1) / ns)) + 4.0f + 0.5f * ns +
-                          2.0f * ns * Q * H * (kDc * 2) / 8e6f);
+        best = {128, std::max(fill, (S + SplitGeom<8, 1>::CHUNK - 1) / SplitGeom<8, 1>::CHUNK), 0};
+        best_us = estimate(128, best.ns);
     }
     for (int hg = 32; hg <= 96 && (S <= kMaxS || best.hg == 0); hg += 32) {
         if (H % hg || (hg == 96 && H % 128 == 0)) continue;  // (96: no 64-bit form)
-        const float start = hg == 32 ? 7.0f : (hg == 64 ? 8.3f : 10.7f);
-        const float tile = hg == 32 ? 1.2f : (hg == 64 ? 1.4f : 1.5f);
         const long wg = (long)Q * (H / hg);
         const int most = scratch ? (int)std::max(1L, std::min({256 / wg, (long)tiles, 64L})) : 1;
         for (int ns = 1; ns <= most; ns++) {
-            const float rounds = (float)((wg * ns + 255) / 256);
-            float us = rounds * (start + tile * ((tiles + ns - 1) / ns));
-            if (ns > 1) us += 4.0f + 0.1f * ns + 2.0f * ns * Q * H * (kDc * 4) / 8e6f;
+            const float us = estimate(hg, ns);
             if (best_us == 0.0f || us < best_us) best = {hg, ns, 0}, best_us = us;
         }
     }
@@ -701,17 +746,22 @@ int launch_dsa_bf16_paged(const uint16_t* qn, const uint16_t* qp, const uint16_t
     AMDMOE_CHECK_ARG(grid < (1L << 31), "dsa_decode_bf16_paged: grid too large");
     float* part_ml = plan.bytes ? (float*)((uint8_t*)scratch + align_up((size_t)Q * ns * H * kDc * (hg == 128 ? 2 : 4), 256))
                                : nullptr;
+    // two token groups from three tiles on (S=64 Q=64 H=32: 9.1 us without, 10.0
+    // with), up to the positions its LDS has room for beside four stages
+    const bool pair = hg == 32 && chunk > 2 * kT32 && chunk <= SplitGeom<2, 2>::CHUNK;
     auto split = hg == 128  ? (wide ? dsa_split_wide_kernel : dsa_split_kernel)
                  : hg == 96 ? dsa_split96_kernel
                  : hg == 64 ? (wide ? dsa_split64_wide_kernel : dsa_split64_kernel)
+                 : pair     ? (wide ? dsa_split32x2_wide_kernel : dsa_split32x2_kernel)
                             : (wide ? dsa_split32_wide_kernel : dsa_split32_kernel);
-    const int lds = hg == 128  ? SplitGeom<8>::LDS
-                    : hg == 96 ? SplitGeom<6>::LDS
-                    : hg == 64 ? SplitGeom<4>::LDS
-                               : SplitGeom<2>::LDS;
+    const int lds = hg == 128  ? SplitGeom<8, 1>::LDS
+                    : hg == 96 ? SplitGeom<6, 1>::LDS
+                    : hg == 64 ? SplitGeom<4, 1>::LDS
+                    : pair     ? SplitGeom<2, 2>::LDS
+                               : SplitGeom<2, 1>::LDS;
     const int rc = ensure_dynamic_lds((const void*)split, lds);
     if (rc != AMDMOE_OK) return rc;
-    hipLaunchKernelGGL(split, dim3((unsigned)grid), dim3(4 * hg), lds, st, qn, qp, cache,
+    hipLaunchKernelGGL(split, dim3((unsigned)grid), dim3(pair ? 256 : 4 * hg), lds, st, qn, qp, cache,
                        cache_tokens * kRowBytes, page_table, logical, out, scratch, part_ml, Q, H, S, page,
                        pages_per_seq, ns, chunk, scale_log2);
     AMDMOE_LAUNCH_CHECK();
