@@ -19,17 +19,26 @@
  *     share one workspace must be ordered on one stream.
  *   - Entry points without a workspace argument that need scratch (the
  *     split-K routing of amdmoe_moe_gate_bf16/_fp8, amdmoe_moe_permute,
- *     amdmoe_dsa_decode_bf16_paged on 128-head groups,
+ *     amdmoe_dsa_decode_bf16_paged with H a multiple of 128,
  *     amdmoe_dsa_indexer_topk_fp8 selecting in parts)
  *     use a per-device buffer of their own family (routing, permutation,
  *     decode, indexer; none is shared with the MoE forward's workspace or
  *     with another family).  A call that must grow that buffer frees and
  *     allocates it, which waits for the device; calls of one family that use
  *     the buffer must be ordered on one stream (concurrent calls of one
- *     family on two streams race on it).  amdmoe_dsa_forward_f32 and the
- *     decode on smaller head groups (H no multiple of 128) may run on any
- *     streams and threads at once: their scratch is one buffer per stream (at
- *     most 8 of at most 64 MiB), and a captured call uses none.
+ *     family on two streams race on it).  A captured call uses that buffer as
+ *     well: make one eager call of the largest size first, as growing later
+ *     would free what the graph uses.
+ *   - amdmoe_dsa_forward_f32 and the decode with H no multiple of 128 may run
+ *     on any streams and threads at once: their scratch is one buffer per
+ *     stream (at most 8 of at most 64 MiB; the call that makes or grows one
+ *     may wait for the device).  A captured call uses none and takes a form
+ *     without: the fp32 attention gives the same bits, slower (Q=8 H=16 Dc=512
+ *     Dp=64 S=1024 336 us for 19); the decode rounds differently than the
+ *     eager call, within its tolerance, and runs one split per query (Q=4 H=64
+ *     S=2000 61 us for 19).  Synchronise a stream that was passed to these two
+ *     before destroying it: another stream may get its handle, and so its
+ *     buffer.
  *   - bf16 tensors are passed as uint16_t (bfloat16 bit patterns), fp8 as
  *     uint8_t OCP e4m3 ("E4M3FN") codes.
  */

@@ -870,22 +870,18 @@ int amdmoe_dsa_decode_bf16_paged(const uint16_t* q_nope, const uint16_t* q_pe,
     const DsaConfig& c = *cfg;
     AMDMOE_CHECK_ARG(c.num_queries >= 0 && c.num_heads >= 1 && c.num_selected_kv >= 1,
                      "bad DsaConfig");
-    // the token-split partials: of 128-head groups in the decode's own cached
-    // scratch, of smaller ones in the stream's, which the call can do without
+    // the splits' partials: where H is a multiple of 128 in the decode's own
+    // cached scratch, captured or not; else in the stream's, which the call
+    // can do without
     DsaPlan plan = dsa_paged_plan(c.num_queries, c.num_heads, c.num_selected_kv, true);
     StreamScratch scr;
     void* scratch = nullptr;
-    if (plan.bytes && plan.hg != 128) {
+    if (plan.bytes && c.num_heads % 128 == 0) {
+        TRY(cached_workspace(plan.bytes, &scratch, SCR_DSA_DECODE));
+    } else if (plan.bytes) {
         TRY(scr.get(plan.bytes, (hipStream_t)stream));
         scratch = scr.ptr;
-        // the plan of a captured call: its scratch grows here already, so
-        // that a call repeated inside a capture need not allocate
-        const DsaPlan bare = dsa_paged_plan(c.num_queries, c.num_heads, c.num_selected_kv, false);
-        void* own = nullptr;
-        if (bare.bytes) TRY(cached_workspace(bare.bytes, &own, SCR_DSA_DECODE));
-        if (!scratch) plan = bare, scratch = own;
-    } else if (plan.bytes) {
-        TRY(cached_workspace(plan.bytes, &scratch, SCR_DSA_DECODE));
+        if (!scratch) plan = dsa_paged_plan(c.num_queries, c.num_heads, c.num_selected_kv, false);
     }
     return launch_dsa_bf16_paged(q_nope, q_pe, cache, c.total_kv_tokens, page_table,
                                  logical_indices, output, c.num_queries, c.num_heads,

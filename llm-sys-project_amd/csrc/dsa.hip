@@ -676,7 +676,7 @@ static float split_us(int hg, int n, float load) {
 // partials.  Head groups of 128 (H a multiple of 128): enough workgroups to
 // cover the chip (256 CUs), at most 2048 tokens per split, at least 32.  Small
 // groups of 32, 64 or 96 heads (S <= 4096): any split that fits the CUs at
-// once, more than one only with stream scratch.  The cheapest by a model
+// once, more than one only with scratch.  The cheapest by a model
 // fitted to measured calls (us): workgroups run in rounds of 256, a merge takes
 // 4 + 0.2 per split (0.5 in the 128-head merge, four splits a round trip) and
 // moves its partials at 8 MB per us (16 where they are bf16).
@@ -689,6 +689,7 @@ DsaPlan dsa_paged_plan(int Q, int H, int S, bool scratch) {
     if (Q < 1 || H < 32 || H % 32 != 0 || S < 1) return best;
     const int tiles = (S + kT32 - 1) / kT32;
     float best_us = 0.0f;
+    int full = 0;  // splits of the 128-head form
     auto estimate = [&](int hg, int ns) {
         const long wgs = (long)Q * (H / hg) * ns;
         const float rounds = (float)((wgs + 255) / 256), load = std::min(1.0f, wgs / 256.0f);
@@ -699,9 +700,10 @@ DsaPlan dsa_paged_plan(int Q, int H, int S, bool scratch) {
     };
     if (H % 128 == 0) {
         const long wg = (long)Q * (H / 128);
-        const int fill = (int)std::min<long>((256 + wg - 1) / wg, tiles);
-        best = {128, std::max(fill, (S + SplitGeom<8, 1>::CHUNK - 1) / SplitGeom<8, 1>::CHUNK), 0};
-        best_us = estimate(128, best.ns);
+        full = (int)std::min<long>((256 + wg - 1) / wg, tiles);
+        full = std::max(full, (S + SplitGeom<8, 1>::CHUNK - 1) / SplitGeom<8, 1>::CHUNK);
+        best = {128, full, 0};
+        best_us = estimate(128, full);
     }
     for (int hg = 32; hg <= 96 && (S <= kMaxS || best.hg == 0); hg += 32) {
         if (H % hg || (hg == 96 && H % 128 == 0)) continue;  // (96: no 64-bit form)
@@ -712,10 +714,16 @@ DsaPlan dsa_paged_plan(int Q, int H, int S, bool scratch) {
             if (best_us == 0.0f || us < best_us) best = {hg, ns, 0}, best_us = us;
         }
     }
-    if (best.hg == 128 || best.ns > 1) {
-        const size_t rows = (size_t)Q * best.ns * H;
-        best.bytes = align_up(rows * kDc * (best.hg == 128 ? 2 : 4), 256) + align_up(rows * 8, 256);
-    }
+    auto bytes = [](size_t rows, int es) { return align_up(rows * kDc * es, 256) + align_up(rows * 8, 256); };
+    if (H % 128 == 0)
+        // The same bytes whatever form runs: the 128-head form's, and at least
+        // what any small groups' splits take (64 heads, 256 workgroups).  The
+        // buffer then grows only where the 128-head form needs more: a buffer
+        // that a call took for granted in a captured graph is not freed by a
+        // smaller call after it.
+        best.bytes = std::max(bytes((size_t)Q * full * H, 2), bytes(256 * 64, 4));
+    else if (best.ns > 1)
+        best.bytes = bytes((size_t)Q * best.ns * H, 4);
     return best;
 }
 

@@ -149,8 +149,8 @@ int launch_dsa_f32(const float* qn, const float* qp, const float* kc, const floa
                    int N, void* scratch, size_t scratch_bytes, hipStream_t st);
 // dsa.hip
 // How a paged decode runs: heads per workgroup, splits per query, bytes of
-// the splits' partials.  hg == 128: in the entry's own scratch; smaller
-// groups: in the stream's, and scratch == false gives a plan without.
+// scratch: for H a multiple of 128 in the entry's own buffer, else of the
+// splits' partials, in the stream's (scratch == false: a plan without).
 struct DsaPlan {
     int hg, ns;
     size_t bytes;

@@ -58,23 +58,52 @@ def test_decode_head_groups(amd, orc, Q, H, S, ctx):
     assert np.abs(got - ref).max() < 1e-2
 
 
-@pytest.mark.parametrize("H", [64, 128])
-def test_decode_groups_streams_and_graph(amd, H):
+def _sets(H, n=3):
     import synth
     Q, S, page = 3, 900, 64
-    sets = [synth.dsa_paged(Q, H, 512, 64, S, page, 1024, seed=s) for s in range(3)]
+    return Q, S, page, [synth.dsa_paged(Q, H, 512, 64, S, page, 1024, seed=s) for s in range(n)]
+
+
+def test_decode_groups_streams(amd):
+    """Calls in flight on several streams at once give the bits of a call alone."""
+    H = 64
+    Q, S, page, sets = _sets(H)
     ref = [_call(amd, t, Q, H, S, page).cpu() for t in sets]
     streams = [torch.cuda.Stream() for _ in range(10)]
     torch.cuda.synchronize()
     outs = []
-    for i in range(30 if H % 128 else 0):
+    for i in range(30):
         with torch.cuda.stream(streams[i % 10]):
             outs.append(_call(amd, sets[i % 3], Q, H, S, page))
     torch.cuda.synchronize()
     for i, o in enumerate(outs):
         assert torch.equal(o.cpu(), ref[i % 3]), i
-    # a captured call has no stream scratch: another split, the same sums in another order
-    out = torch.empty_like(ref[0], device="cuda")
+
+
+def test_decode_groups_in_turn(amd):
+    """H a multiple of 128: calls of changing inputs and sizes one after the
+    other on one stream, which share their scratch."""
+    import synth
+    shapes = [(3, 128, 900), (1, 128, 2048), (64, 128, 64), (2, 256, 513), (40, 128, 700)]
+    ts = [(q, h, s, synth.dsa_paged(q, h, 512, 64, s, 64, 2048, seed=q + s)) for q, h, s in shapes]
+    ref = []
+    for q, h, s, t in ts:
+        ref.append(_call(amd, t, q, h, s, 64).cpu())
+        torch.cuda.synchronize()
+    order = [0, 1, 0, 2, 1, 3, 4, 3, 0, 4, 2, 1]
+    outs = [_call(amd, ts[i][3], *ts[i][:3], 64) for i in order]
+    torch.cuda.synchronize()
+    for i, o in zip(order, outs):
+        assert torch.equal(o.cpu(), ref[i]), i
+
+
+@pytest.mark.parametrize("H", [64, 128])
+def test_decode_groups_graph(amd, H):
+    """A captured call: H a multiple of 128 runs the eager call's plan, with the
+    same bits; otherwise one split (no scratch), the same sums in another order."""
+    Q, S, page, sets = _sets(H)
+    ref = _call(amd, sets[0], Q, H, S, page).cpu()
+    out = torch.empty_like(ref, device="cuda")
     cfg = amd.dsa_config(Q, H, 512, 64, S, page, sets[0][2].shape[0])
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
@@ -84,5 +113,7 @@ def test_decode_groups_streams_and_graph(amd, H):
         _call(amd, sets[1], Q, H, S, page)
         g.replay()
         torch.cuda.synchronize()
-        d = (out.cpu().view(torch.bfloat16).float() - ref[0].view(torch.bfloat16).float()).abs().max()
+        if H % 128 == 0:
+            assert torch.equal(out.cpu(), ref)
+        d = (out.cpu().view(torch.bfloat16).float() - ref.view(torch.bfloat16).float()).abs().max()
         assert d < 1e-2
