@@ -31,8 +31,9 @@
  *     would free what the graph uses.
  *   - amdmoe_dsa_forward_f32 and the decode with H no multiple of 128 may run
  *     on any streams and threads at once: their scratch is one buffer per
- *     stream (at most 8 of at most 64 MiB; the call that makes or grows one
- *     may wait for the device).  A captured call uses none and takes a form
+ *     stream (at most 256 of at most 64 MiB, 4 GiB together; the call that
+ *     makes or grows one may wait for the device, and a call past these
+ *     bounds allocates and frees in stream order).  A captured call uses none and takes a form
  *     without: the fp32 attention gives the same bits, slower (Q=8 H=16 Dc=512
  *     Dp=64 S=1024 336 us for 19); the decode rounds differently than the
  *     eager call, within its tolerance, and runs one split per query (Q=4 H=64

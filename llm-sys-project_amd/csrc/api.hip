@@ -167,19 +167,25 @@ static int cached_workspace(size_t need, void** out, int kind = SCR_MOE) {
 
 // Scratch of calls that may run on any streams and threads at once and
 // inside a graph capture: one buffer per (device, stream), at most
-// kStreamSlots of them (the least recently used one goes first; hipFree
-// waits for the device, so for what still reads it) and never more than
-// kStreamScratchMax bytes each.  A new stream may get a destroyed one's
-// handle and so its buffer: hipStreamDestroy waits for the stream's work
-// (measured with a kernel of 167 ms).  The lock is held from get() until the
-// object dies, so that the launches of one call that share the buffer are
-// enqueued next to each other.  While the stream is being captured there is
-// no scratch (a graph may outlive the buffer and be replayed on any stream),
-// nor when it cannot be allocated: ptr stays null and the caller takes its
-// form that needs none.  (hipMallocAsync / hipFreeAsync around the launches
-// cost 13 us of host time per call, an event per call 4 us.)
-constexpr int kStreamSlots = 8;
-constexpr size_t kStreamScratchMax = 64u << 20;
+// kStreamSlots of them, of at most kStreamScratchMax bytes each and
+// kStreamScratchSum together.  A buffer is freed for another stream's only
+// after kStreamIdle calls that did not use it (hipFree waits for the device, so
+// for what still reads it); until then a stream past these bounds allocates
+// and frees in stream order (13 us of host time per call, and the runtime may
+// wait for memory that another stream has freed but not finished with).
+// (Eight slots that gave way at once made every call of nine streams wait for
+// the device.)  A new stream may get a
+// destroyed one's handle and so its buffer: the caller synchronises a stream
+// before it destroys it (amdmoe.h; the runtimes measured wait in
+// hipStreamDestroy, but HIP does not promise it).  The lock is held from get()
+// until the object dies, so that the launches of one call that share the
+// buffer are enqueued next to each other.  While the stream is being captured
+// there is no scratch (a graph may outlive the buffer and be replayed on any
+// stream), nor when it cannot be allocated: ptr stays null and the caller takes
+// its form that needs none.
+constexpr int kStreamSlots = 256;
+constexpr unsigned long long kStreamIdle = 4096;
+constexpr size_t kStreamScratchMax = 64u << 20, kStreamScratchSum = (size_t)4 << 30;
 struct StreamSlot {
     int dev = -1;
     hipStream_t st = nullptr;
@@ -196,6 +202,7 @@ class StreamScratch {
         static std::mutex mu;
         static StreamSlot slots[kStreamSlots];
         static unsigned long long clock = 0;
+        static size_t sum = 0;  // bytes of all slots
         if (need == 0 || need > kStreamScratchMax) return AMDMOE_OK;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
@@ -215,33 +222,20 @@ class StreamScratch {
         lock_ = std::unique_lock<std::mutex>(mu);
         StreamSlot* s = nullptr;
         for (StreamSlot& c : slots)
-            if (c.ptr && c.dev == dev && c.st == st && c.thread == thread) s = &c;
+            if (c.ptr && c.dev == dev && c.st == st && c.thread == thread) {
+                s = &c;
+                break;
+            }
         if (!s || s->bytes < need) {
             // another thread's capture must not see the allocation
             hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
             AMDMOE_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-            if (!s) {
-                s = &slots[0];
-                for (StreamSlot& c : slots)
-                    if (c.used < s->used) s = &c;
-            }
-            int rc = free_slot(*s);
-            if (rc == AMDMOE_OK) {
-                const size_t grow = std::min(kStreamScratchMax, align_up(need + need / 4, 1 << 20));
-                if (hipMalloc(&s->ptr, grow) == hipSuccess) {
-                    s->dev = dev, s->st = st, s->thread = thread, s->bytes = grow;
-                } else {
-                    (void)hipGetLastError();
-                    s->ptr = nullptr;
-                }
-            }
-            const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
-            if (rc != AMDMOE_OK) return rc;
-            AMDMOE_HIP_TRY(back);
-            if (!s->ptr) {
-                *s = StreamSlot();
+            const int rc = make(slots, sum, clock, need, dev, st, thread, s);
+            AMDMOE_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+            if (rc != AMDMOE_OK || !s) {
+                ++clock;
                 lock_.unlock();
-                return AMDMOE_OK;
+                return rc;
             }
         }
         s->used = ++clock;
@@ -250,14 +244,58 @@ class StreamScratch {
         return AMDMOE_OK;
     }
 
+    StreamScratch() = default;
+    StreamScratch(const StreamScratch&) = delete;
+    ~StreamScratch() {
+        if (ordered_ && hipFreeAsync(ordered_, st_) != hipSuccess) (void)hipGetLastError();
+    }
+
   private:
-    static int free_slot(StreamSlot& s) {
-        if (!s.ptr) return AMDMOE_OK;
+    void* ordered_ = nullptr;  // allocated in the order of st_, freed behind the launches
+    hipStream_t st_ = nullptr;
+    // A buffer of `need` bytes: s becomes its slot, or null where the call's own
+    // allocation (ordered_) or none serves.
+    int make(StreamSlot (&slots)[kStreamSlots], size_t& sum, unsigned long long clock, size_t need, int dev,
+             hipStream_t st, unsigned long long thread, StreamSlot*& s) {
+        const size_t grow = std::min(kStreamScratchMax, align_up(need + need / 4, 1 << 20));
+        int rc = s ? free_slot(*s, sum) : AMDMOE_OK;
+        for (; rc == AMDMOE_OK;) {
+            StreamSlot *empty = nullptr, *old = nullptr;
+            for (StreamSlot& c : slots)
+                if (!c.ptr) empty = empty ? empty : &c;
+                else if (!old || c.used < old->used) old = &c;
+            s = empty;
+            if (s && sum + grow <= kStreamScratchSum) break;
+            if (clock - old->used < kStreamIdle) {  // all in use
+                s = nullptr;
+                if (hipMallocAsync(&ordered_, need, st) == hipSuccess) {
+                    ptr = ordered_, bytes = need, st_ = st;
+                } else {
+                    (void)hipGetLastError();
+                    ordered_ = nullptr;
+                }
+                return AMDMOE_OK;
+            }
+            rc = free_slot(*old, sum);
+        }
+        if (rc != AMDMOE_OK) return rc;
+        if (hipMalloc(&s->ptr, grow) != hipSuccess) {
+            (void)hipGetLastError();
+            *s = StreamSlot();
+            s = nullptr;
+            return AMDMOE_OK;
+        }
+        s->dev = dev, s->st = st, s->thread = thread, s->bytes = grow;
+        sum += grow;
+        return AMDMOE_OK;
+    }
+    static int free_slot(StreamSlot& s, size_t& sum) {
         int cur = 0;
         AMDMOE_HIP_TRY(hipGetDevice(&cur));
         if (s.dev != cur) AMDMOE_HIP_TRY(hipSetDevice(s.dev));
         const hipError_t e = hipFree(s.ptr);
         if (s.dev != cur) AMDMOE_HIP_TRY(hipSetDevice(cur));
+        sum -= s.bytes;
         s = StreamSlot();
         AMDMOE_HIP_TRY(e);
         return AMDMOE_OK;

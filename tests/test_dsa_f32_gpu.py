@@ -99,6 +99,41 @@ def test_dsa_f32_streams_and_graph(amd):
         assert torch.equal(out.cpu(), ref[0])
 
 
+@pytest.mark.parametrize("n", [12, 70])
+def test_dsa_f32_many_streams(amd, n):
+    """Streams in turn, up to more than there are scratch buffers: the same bits,
+    and once each has had its first call none waits for the device."""
+    import ctypes
+    shape = (2, 8, 64, 16, 500, 1024)
+    t = [torch.from_numpy(x).cuda() for x in _inputs(*shape, seed=4)]
+    ref = _run(amd, t, shape).cpu()
+    lib = amd.load()
+    raw = []
+    for _ in range(n):
+        p = ctypes.c_void_p()
+        assert lib.hipStreamCreateWithFlags(ctypes.byref(p), 1) == 0  # non-blocking
+        raw.append(p)
+    streams = [torch.cuda.ExternalStream(p.value) for p in raw]
+    cfg = amd.dsa_config(*shape[:5], 16, shape[5])
+    outs = [torch.empty_like(t[0]) for _ in streams]
+    side, done = torch.cuda.Stream(), torch.cuda.Event()
+    torch.cuda.synchronize()
+    for turn in range(3):
+        if turn == 1:  # every stream has had a call
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(200_000_000)
+                done.record()
+        for s, out in zip(streams, outs):
+            amd.dsa_forward_f32(*t, out, cfg, s)
+    assert not done.query()
+    torch.cuda.synchronize()
+    for out in outs:
+        assert torch.equal(out.cpu(), ref)
+    for p in raw:
+        assert lib.hipStreamDestroy(p) == 0
+
+
 def test_dsa_f32_non_finite(amd):
     """As in the reference's loops: a NaN or +inf score makes its head NaN, a
     head without a score above -inf (all -inf, or all NaN) gives 0; an infinity

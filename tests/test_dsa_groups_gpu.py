@@ -64,20 +64,30 @@ def _sets(H, n=3):
     return Q, S, page, [synth.dsa_paged(Q, H, 512, 64, S, page, 1024, seed=s) for s in range(n)]
 
 
-def test_decode_groups_streams(amd):
-    """Calls in flight on several streams at once give the bits of a call alone."""
+@pytest.mark.parametrize("n", [10, 280])
+def test_decode_groups_streams(amd, n):
+    """Calls in flight on several streams at once, up to more than there are
+    scratch buffers, give the bits of a call alone."""
+    import ctypes
     H = 64
     Q, S, page, sets = _sets(H)
     ref = [_call(amd, t, Q, H, S, page).cpu() for t in sets]
-    streams = [torch.cuda.Stream() for _ in range(10)]
+    lib = amd.load()
+    raw = [ctypes.c_void_p() for _ in range(n)]
+    for p in raw:
+        assert lib.hipStreamCreateWithFlags(ctypes.byref(p), 1) == 0  # non-blocking
+    streams = [torch.cuda.ExternalStream(p.value) for p in raw]
+    outs = [torch.empty_like(ref[0], device="cuda") for _ in range(3 * n)]
+    cfg = amd.dsa_config(Q, H, 512, 64, S, page, sets[0][2].shape[0])
     torch.cuda.synchronize()
-    outs = []
-    for i in range(30):
-        with torch.cuda.stream(streams[i % 10]):
-            outs.append(_call(amd, sets[i % 3], Q, H, S, page))
+    for i, out in enumerate(outs):
+        t = sets[i % 3]
+        amd.dsa_decode_bf16_paged(*t[:5], out, cfg, t[5], streams[i % n])
     torch.cuda.synchronize()
     for i, o in enumerate(outs):
         assert torch.equal(o.cpu(), ref[i % 3]), i
+    for p in raw:
+        assert lib.hipStreamDestroy(p) == 0
 
 
 def test_decode_groups_in_turn(amd):
