@@ -13,7 +13,9 @@
 //       straight from memory, 16 bytes per lane (a K row is used once per
 //       16 heads, so staging it would only add a pass); the 8 waves split
 //       the chunk's token tiles, and the columns when there are fewer tiles
-//   p = expf(s - m) with the chunk's max m, l = sum p, in LDS
+//   p = expf(s - m) 2^-k with the chunk's max m, l = sum p, in LDS; 2^k >= n
+//       keeps every partial sum of p V within max |V| (the reference divides
+//       before it sums) and divides out exactly at the end
 //   O^T (64 dims x 16 heads) += V^T . P^T  16x16x4 fp32; the 8 waves split
 //       the 64-dim blocks, and the tokens when there are fewer blocks
 // and the chunks' (m, l, O) are folded in order with the usual rescaling:
@@ -174,11 +176,11 @@ __device__ __forceinline__ void f32_pv_load(const DsaF32Args& a, const DsaF32Lds
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// (m, l) of a chunk of len (1 .. kF32Max) positions whose rows are in
-// L.rows: leaves p = expf(s - m) in L.p, zero past len.  The first V loads
+// (m, l) of a chunk of len (1 .. kF32Max) of the query's n positions, its rows
+// in L.rows: leaves p = expf(s - m) 2^-k in L.p, zero past len.  The first V loads
 // of f32_pv go out (into vv) once the K loads have, under the softmax.
 template <bool VEC>
-__device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, int qi, int h0, int len,
+__device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, int qi, int h0, int n, int len,
                                            float scale, f32x4 (&vv)[kPvB]) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -242,10 +244,11 @@ __device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, in
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
     const float mu = mx == -INFINITY ? 0.0f : mx;  // every score -inf: p = 0
+    const float pn = __int_as_float((95 + __clz(n - 1)) << 23);  // 2^-k, k = 32 - clz(n - 1)
     float sum = 0.0f;
 #pragma unroll 1
     for (int t = j; t < 16 * nt; t += 32) {
-        const float p = t < len ? expf(ph[t] - mu) : 0.0f;
+        const float p = t < len ? expf(ph[t] - mu) * pn : 0.0f;
         ph[t] = p;
         sum += p;
     }
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(512) void f32_split_kernel(DsaF32Args a) {
     }
     const int len = min(chunk, n - c0);
     f32x4 vv[kPvB];
-    f32_scores<VEC>(a, L, qi, h0, len, 1.0f / sqrtf((float)(a.Dc + a.Dp)), vv);
+    f32_scores<VEC>(a, L, qi, h0, n, len, 1.0f / sqrtf((float)(a.Dc + a.Dp)), vv);
     if (threadIdx.x < 16) a.part_ml[slot + threadIdx.x] = make_float2(L.m[threadIdx.x], L.l[threadIdx.x]);
     f32_pv<VEC>(a, L, len, vv, [&](int hd, int d, f32x4 o) __attribute__((always_inline)) {
         if (h0 + hd < a.H) store4<VEC>(a.part_o + (slot + hd) * a.Dc, d, a.Dc, o);
@@ -454,7 +457,7 @@ __global__ __launch_bounds__(512) void f32_loop_kernel(DsaF32Args a) {
         }
         const int len = min(chunk, n - c0);
         f32x4 vv[kPvB];
-        f32_scores<VEC>(a, L, qi, h0, len, scale, vv);
+        f32_scores<VEC>(a, L, qi, h0, n, len, scale, vv);
         if (tid < 16) {
             float m = s_m[tid], l = s_l[tid];
             s_f[tid] = f32_fold(m, l, L.m[tid], L.l[tid]);

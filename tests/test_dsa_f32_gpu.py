@@ -99,6 +99,20 @@ def test_dsa_f32_streams_and_graph(amd):
         assert torch.equal(out.cpu(), ref[0])
 
 
+@pytest.mark.parametrize("shape", [(1, 2, 64, 16, 100, 256), (2, 4, 64, 16, 300, 512), (1, 2, 7, 3, 1500, 2000),
+                                   (65, 64, 40, 8, 140, 256)], ids=["chunk", "split", "split-scalar", "loop"])
+def test_dsa_f32_largest_values(amd, orc, shape):
+    """V near the largest float: the output is an average of its rows (the
+    reference divides the probabilities before it sums), so it is finite.  5e-6
+    of it: the probabilities' and the sums' rounding."""
+    a = list(_inputs(*shape, seed=11))
+    a[4] = (np.float32(3.3e38) * np.sign(a[4][:1]) * (1.0 - np.abs(a[4]) / 10)).astype(np.float32)
+    ref = orc.dsa_forward_f32(*a)
+    assert np.isfinite(ref).all()
+    out = _run(amd, [torch.from_numpy(x).cuda() for x in a], shape).cpu().numpy()
+    assert np.abs(out / ref - 1.0).max() < 5e-6
+
+
 @pytest.mark.parametrize("n", [12, 70])
 def test_dsa_f32_many_streams(amd, n):
     """Streams in turn, up to more than there are scratch buffers: the same bits,
