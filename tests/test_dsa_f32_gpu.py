@@ -113,6 +113,32 @@ def test_dsa_f32_largest_values(amd, orc, shape):
     assert np.abs(out / ref - 1.0).max() < 5e-6
 
 
+@pytest.mark.parametrize("shape,valid", [((1, 1, 8, 4, 5000, 5000), "all"), ((260, 1, 8, 4, 5000, 5000), "all"),
+                                         ((260, 1, 8, 4, 5000, 5000), "tail"), ((260, 1, 8, 4, 5000, 5000), "sparse"),
+                                         ((260, 1, 8, 4, 20000, 20000), "gaps"), ((2, 1, 8, 4, 20000, 20000), "gaps")],
+                         ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_dsa_f32_long_lists(amd, orc, shape, valid):
+    """Selections of many chunks (the windows' cursor): every position, only the
+    last ones, one in 7, and lists with whole segments invalid."""
+    Q, H, Dc, Dp, S, N = shape
+    a = list(_inputs(*shape, seed=S + Q))
+    a[5][:] = np.arange(S)[None]
+    keep = np.zeros(S, bool)
+    if valid == "all":
+        keep[:] = True
+    elif valid == "tail":
+        keep[S - 700:] = True
+    elif valid == "sparse":
+        keep[3::7] = True
+    else:
+        keep[:64] = keep[S // 8 - 1: S // 8 + 70] = keep[S // 2: S // 2 + 3000] = keep[-1:] = True
+    a[5][:, ~keep] = -1
+    out = _run(amd, [torch.from_numpy(x).cuda() for x in a], shape).cpu().numpy()
+    for q in sorted({0, Q // 2, Q - 1}):
+        ref = orc.dsa_forward_f32(a[0][q:q + 1], a[1][q:q + 1], a[2], a[3], a[4], a[5][q:q + 1][:, keep])
+        assert np.abs(out[q] - ref[0]).max() < 1e-6
+
+
 @pytest.mark.parametrize("n", [12, 70])
 def test_dsa_f32_many_streams(amd, n):
     """Streams in turn, up to more than there are scratch buffers: the same bits,
