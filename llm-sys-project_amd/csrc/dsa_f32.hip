@@ -512,13 +512,14 @@ static size_t f32_query_bytes(int H, int Dc, int S) {  // partials of one query
     const size_t slots = (size_t)((H + 15) / 16) * f32_max_chunks(S) * 16;
     return slots * Dc * 4 + slots * 8;
 }
-constexpr size_t kF32Scratch = 64u << 20;  // queries are taken in groups whose partials fit this
+constexpr size_t kF32Pad = 512;                      // the (m, l) pairs' alignment
+constexpr size_t kF32Scratch = (64u << 20) - kF32Pad;  // queries are taken in groups whose partials fit this
 
 size_t dsa_f32_scratch_bytes(int Q, int H, int Dc, int S) {
     if (Q < 1 || H < 1 || f32_max_chunks(S) == 1 || f32_head_tiles(Q, H) >= 256) return 0;
     const size_t one = f32_query_bytes(H, Dc, S);
     const size_t group = std::max<size_t>(1, std::min<size_t>(Q, kF32Scratch / one));
-    return one > kF32Scratch ? 0 : group * one + 512;
+    return one > kF32Scratch ? 0 : group * one + kF32Pad;
 }
 
 template <bool VEC>
@@ -532,7 +533,7 @@ static int launch_f32(DsaF32Args a, int Q, void* scratch, size_t scratch_bytes, 
     }
     const int ht = (a.H + 15) / 16, nd = (a.Dc + 63) / 64;
     a.nc = f32_max_chunks(a.S);
-    const int group = (int)std::min<size_t>(Q, (scratch_bytes - 512) / f32_query_bytes(a.H, a.Dc, a.S));
+    const int group = (int)std::min<size_t>(Q, (scratch_bytes - kF32Pad) / f32_query_bytes(a.H, a.Dc, a.S));
     AMDMOE_CHECK_ARG(group >= 1, "dsa_forward: scratch of %zu bytes", scratch_bytes);
     const size_t slots = (size_t)group * ht * a.nc * 16;
     a.part_o = (float*)scratch;

@@ -124,3 +124,17 @@ def test_pack_weights_bf16_validates_before_device_work():
     cfg = amdmoe.moe_config(4, 4, 2, 64, 128)
     rc = lib.amdmoe_moe_forward_bf16_packed(None, None, None, None, None, None, ctypes.byref(cfg), None, 0, None)
     assert rc == 1 and b"null" in lib.amdmoe_last_error()
+
+
+def test_fp32_attention_scratch_fits_a_stream_buffer():
+    """The chunks' partials are asked for in groups of queries that fit the
+    64 MiB of one stream's buffer (more is never given: the call would fall
+    back to its slow form), wherever one query's fit."""
+    fn = ctypes.CDLL(amdmoe.LIB_PATH)._ZN6amdmoe21dsa_f32_scratch_bytesEiiii
+    fn.restype, fn.argtypes = ctypes.c_size_t, [ctypes.c_int] * 4
+    for Q in (1, 7, 63, 64, 100, 255):
+        for H in (1, 16, 17):
+            for Dc in (1, 62, 126, 254, 255, 510, 512, 1022, 2046):
+                for S in (129, 1000, 1024, 8192):
+                    if Q * ((H + 15) // 16) < 256:
+                        assert 0 < fn(Q, H, Dc, S) <= 64 << 20, (Q, H, Dc, S)
