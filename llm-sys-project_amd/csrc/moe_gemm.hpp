@@ -190,7 +190,6 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
     // scale byte); a wave whose activation rows are all past the live token
     // tiles issues only the weight loads
     static_assert(DT == DT_FP8 || DT == DT_MX, "fp32 and bf16 have kernels of their own");
-    constexpr bool kScaledA = true;  // activations carry row scales
     static_assert(DT != DT_MX || PK, "MX weights exist in fragment order only");
     using Frag = std::conditional_t<DT == DT_MX, BFragMx, BFrag>;
     // per K-step and wave: ceil(R/4) activation slabs of 8 rows (the 2R slabs
@@ -217,24 +216,20 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
     const int4 tile0 = g.tiles[mt0];
     const int m_tiles = tile0.w & 0xffff, first_tile = mt0 - (tile0.w >> 16);
     const int l_item = w - first_tile * ntn;
-    const int ntv = __builtin_amdgcn_readfirstlane(l_item / m_tiles);
-    const int mt = first_tile + (l_item - ntv * m_tiles);
-    const int nt = ntv;
+    const int nt = __builtin_amdgcn_readfirstlane(l_item / m_tiles);
+    const int mt = first_tile + (l_item - nt * m_tiles);
     const int4 tile = m_tiles == 1 ? tile0 : g.tiles[mt];
     // uniform values (SGPRs): the asm loads take their soffsets from them
     const int e = __builtin_amdgcn_readfirstlane(tile.x), row0 = __builtin_amdgcn_readfirstlane(tile.y),
               rows = __builtin_amdgcn_readfirstlane(tile.z);
-    const int nk_all = (int)((long)g.K * ES / 128);  // K-steps of the whole reduction
-    const int nk = nk_all;
+    const int nk = (int)((long)g.K * ES / 128);  // K-steps
     const int kb_per_row = g.K / 128;  // fp8 scale blocks along K
 
     // ---- buffer descriptors ----
     const uint8_t* bexp = g.b + (size_t)e * g.b_expert_bytes;
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(g.a, g.a_bytes);
     const i32x4 rb = make_rsrc_words(bexp, g.b_expert_bytes);
-    const __amdgpu_buffer_rsrc_t rs =
-        make_rsrc(kScaledA ? (const void*)g.a_scale : (const void*)g.a,
-                  kScaledA ? g.a_scale_bytes : 0);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(g.a_scale, g.a_scale_bytes);
     const i32x4 rbs = DT == DT_MX ? make_rsrc_words(g.b_mx_scale + (size_t)e * g.b_mx_scale_expert_bytes,
                                                     g.b_mx_scale_expert_bytes)
                                   : rb;
@@ -295,10 +290,7 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
     // wave's scale slot are one 128-byte line (row-major, every gathered
     // row's scale was a line of its own: UP 8% slower)
     uint32_t voff_s = kOob;
-    if (kScaledA) {
-        const int r = 32 * wave + lane;
-        if (lane < 32 && r < rows) voff_s = (uint32_t)((row0 + r) * 4);
-    }
+    if (const int r = 32 * wave + lane; lane < 32 && r < rows) voff_s = (uint32_t)((row0 + r) * 4);
     const int scale_kstride = (int)(g.a_scale_rows * 4);  // bytes per K-step of a_scale
 
     // ---- weight rows of this wave: two MFMA column tiles of 16 ----
@@ -323,7 +315,7 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
         const long nb = PK ? (n - r16) * g.b_row_bytes + 16 * lane : n * g.b_row_bytes + 16 * q;
         voff_b[ct] = ok ? (uint32_t)nb : kOob;
         // MX: E8M0 scales of the 16 rows' K-step, [lane] bytes per block of 64
-        voff_bs[ct] = ok ? (uint32_t)((n - r16) / 16 * nk_all * 64 + lane) : kOob;
+        voff_bs[ct] = ok ? (uint32_t)((n - r16) / 16 * nk * 64 + lane) : kOob;
     }
     __builtin_amdgcn_sched_barrier(0);
     int row_slot = 0;
@@ -381,9 +373,9 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
                           int so_v, uint8_t* st_, Frag& f, u32x4 (&av)[4]) __attribute__((always_inline)) {
         constexpr int R = decltype(rc)::value;
         constexpr int NS = (R + 3) / 4;
-        constexpr int kAS = NS + (kScaledA ? 1 : 0);
+        constexpr int kAS = NS + 1;
         if (sl < NS) {
-            if constexpr ((kScaledA && R <= (DT == DT_MX ? kVgMaxRMx : kVgMaxR)) || (DT == DT_FP8 && R > kVgMaxR))  // register path: K-step KT_V into av
+            if constexpr (R <= (DT == DT_MX ? kVgMaxRMx : kVgMaxR) || (DT == DT_FP8 && R > kVgMaxR))  // register path: K-step KT_V into av
                 av[sl < 4 ? sl : 0] = buffer_load_b128_async<0>(rv_, voff_a[sl], so_v);
             else
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -439,10 +431,8 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
             const u32x4 lo = *(const u32x4*)(p + off_lo), hi = *(const u32x4*)(p + off_hi);
             xv = (i32x8){(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
                          (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-            if (kScaledA) {  // fp8: the row's fp32 scale; MX: its four E8M0 bytes
-                const int r = 16 * rt + r16;
-                sx = *(const float*)(base + kATile + (r >> 5) * 256 + (r & 31) * 4);
-            }
+            const int r = 16 * rt + r16;  // fp8: the row's fp32 scale; MX: its four E8M0 bytes
+            sx = *(const float*)(base + kATile + (r >> 5) * 256 + (r & 31) * 4);
         };
         auto mma = [&](int rt, const i32x8& xv, float sx) __attribute__((always_inline)) {
             if constexpr (DT == DT_MX) {
@@ -536,8 +526,8 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
         constexpr int R = decltype(rc)::value;  // token tiles per step
         constexpr int RB = decltype(rbc)::value;
         constexpr int NS = (R + 3) / 4;
-        constexpr int kSl = NS + (kScaledA ? 1 : 0) + 4;
-        constexpr bool kVg = kScaledA && R <= (DT == DT_MX ? kVgMaxRMx : kVgMaxR);
+        constexpr int kSl = NS + 5;
+        constexpr bool kVg = R <= (DT == DT_MX ? kVgMaxRMx : kVgMaxR);
         constexpr bool kVg1 = DT == DT_FP8 && R > kVgMaxR;  // one register set (MX: registers run out)
         // Issue order per step: activation slots of step kt+2, then the 4
         // weight loads of step kt+RB-1.  Everything of step kt has landed
@@ -601,7 +591,7 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
             for (int j = 0; j < 2; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         Frag bs[RB];
         constexpr int NS = (R + 3) / 4;
-        constexpr bool kVg = kScaledA && R <= (DT == DT_MX ? kVgMaxRMx : kVgMaxR);
+        constexpr bool kVg = R <= (DT == DT_MX ? kVgMaxRMx : kVgMaxR);
         constexpr bool kVg1 = DT == DT_FP8 && R > kVgMaxR;
         u32x4 av[2][4];  // register path: activations of odd / even K-steps (kVg1: set 0 only)
         if constexpr (kVg1) {
@@ -657,7 +647,7 @@ __global__ __launch_bounds__(512, 1) void grouped_gemm_kernel(GemmArgs g) {
             // 0..RB-2)
             static_for<(RB - 1 > 2 ? RB - 1 : 2)>([&](auto ic) __attribute__((always_inline)) {
                 constexpr int i = decltype(ic)::value;
-                constexpr int kAS = NS + (kScaledA ? 1 : 0);
+                constexpr int kAS = NS + 1;
                 STEP_ADDR(i, i, i);
                 for (int sl = 0; sl < kAS + 4; sl++)
                     if (sl < kAS ? i < 2 : i < RB - 1) issue_slot(rc, sl, SLOT_ARGS, bs[i < RB ? i : 0], av[0]);

@@ -138,3 +138,14 @@ def test_fp32_attention_scratch_fits_a_stream_buffer():
                 for S in (129, 1000, 1024, 8192):
                     if Q * ((H + 15) // 16) < 256:
                         assert 0 < fn(Q, H, Dc, S) <= 64 << 20, (Q, H, Dc, S)
+
+
+def test_shared_grouped_gemm_refuses_fp32():
+    """The fp32 layer has kernels of its own: the shared launcher, which picks
+    among the bf16 / fp8 / MX ones, must not run fp32 operands as fp8."""
+    lib = ctypes.CDLL(amdmoe.LIB_PATH)
+    fn = lib._ZN6amdmoe19launch_grouped_gemmEiiRKNS_8GemmArgsElP12ihipStream_t
+    fn.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p]
+    lib.amdmoe_last_error.restype = ctypes.c_char_p
+    args = ctypes.create_string_buffer(1024)  # a zeroed GemmArgs; no tiles, so nothing would be launched
+    assert fn(0, 0, args, 0, None) == 1 and b"dtype 0" in lib.amdmoe_last_error()
