@@ -166,11 +166,12 @@ __device__ __forceinline__ unsigned wave_prefix_sum(unsigned x, int lane) {
 // 32768]: 60.0 us with 12 workgroups per query, which wait for the longest,
 // 53.6 with equal runs).  A run that reaches the next query loads that query's
 // heads on the way.  Otherwise workgroup (query, part) takes tiles part,
-// part + nparts, ...
+// part + nparts, ...  Both forms run 4 waves per SIMD up to 32 heads, 3 to 64, 2 to
+// 128.
 constexpr int kIdxBalanced = 256;
 
 template <int HT, bool POW2, bool EVEN>  // head tiles of 16; page size a power of two (2^shift)
-__global__ __launch_bounds__(256) void indexer_scores_kernel(
+__global__ __launch_bounds__(256, EVEN && HT <= 2 ? 4 : 1) void indexer_scores_kernel(
     const uint8_t* __restrict__ qc, const float* __restrict__ qs, const float* __restrict__ hw,
     const uint8_t* __restrict__ kc, long kc_bytes, const float* __restrict__ ks,
     const int* __restrict__ page_table, const int* __restrict__ seq_len, int Q, int page, int shift,
@@ -231,44 +232,42 @@ __global__ __launch_bounds__(256) void indexer_scores_kernel(
         if (qi < Q) score(qi, [&]() { return min(seq_len[qi], cap); }, part, nparts, ntile);
         return;
     }
-    // tiles up to and including each query, by 64 queries (lane's query 64k + lane)
-    unsigned incl[kIdxBalanced / 64];
-    int lens[kIdxBalanced / 64];
-#pragma unroll
-    for (int k = 0; k < kIdxBalanced / 64; k++) lens[k] = 64 * k + lane < Q ? min(seq_len[64 * k + lane], cap) : 0;
+    // each query's positions and the tiles up to and including it, in LDS (in
+    // registers they live through the scoring loop: 10 more, a wave per SIMD less
+    // at 32 heads and fewer)
+    __shared__ int s_len[kIdxBalanced];
+    __shared__ unsigned s_incl[kIdxBalanced];
     unsigned total = 0;
+    {
+        int lens[kIdxBalanced / 64];
 #pragma unroll
-    for (int k = 0; k < kIdxBalanced / 64; k++) {
-        incl[k] = total + wave_prefix_sum((unsigned)(max(lens[k], 0) + kIdxTile - 1) / kIdxTile, lane);
-        total = __builtin_amdgcn_readlane(incl[k], 63);
+        for (int k = 0; k < kIdxBalanced / 64; k++)
+            lens[k] = 64 * k + lane < Q ? max(min(seq_len[64 * k + lane], cap), 0) : 0;
+#pragma unroll
+        for (int k = 0; k < kIdxBalanced / 64; k++) {
+            const unsigned incl = total + wave_prefix_sum((unsigned)(lens[k] + kIdxTile - 1) / kIdxTile, lane);
+            total = __builtin_amdgcn_readlane(incl, 63);
+            if (wave == 0) s_len[64 * k + lane] = lens[k], s_incl[64 * k + lane] = incl;
+        }
     }
+    __syncthreads();
     unsigned at = (unsigned)((unsigned long)total * blockIdx.x / gridDim.x);
     const unsigned end = (unsigned)((unsigned long)total * (blockIdx.x + 1) / gridDim.x);
     while (at < end) {
         int qi = 0;  // the queries whose tiles lie before `at`
 #pragma unroll
         for (int k = 0; k < kIdxBalanced / 64; k++)
-            if (64 * k < Q) qi += __popcll(__ballot(incl[k] <= at && 64 * k + lane < Q));
-        unsigned upto = 0;
-        int len = 0;
-#pragma unroll
-        for (int k = 0; k < kIdxBalanced / 64; k++)
-            if (qi >> 6 == k) {
-                upto = __builtin_amdgcn_readlane(incl[k], qi & 63);
-                len = __builtin_amdgcn_readlane(lens[k], qi & 63);
-            }
+            if (64 * k < Q) qi += __popcll(__ballot(s_incl[64 * k + lane] <= at && 64 * k + lane < Q));
+        const unsigned upto = __builtin_amdgcn_readfirstlane(s_incl[qi]);
+        const int len = __builtin_amdgcn_readfirstlane(s_len[qi]);
         const unsigned first = upto - (unsigned)(len + kIdxTile - 1) / kIdxTile;  // of this query
         const unsigned stop = min(end, upto);
         score(qi, [&]() { return len; }, (int)(at - first), 1, (int)(stop - first));
         at = stop;
     }
-    // the positions past the last live tiles, by all workgroups
+    // the positions past each query's last live tile, a query per workgroup
     for (int qi = blockIdx.x; qi < Q; qi += gridDim.x) {
-        int len = 0;
-#pragma unroll
-        for (int k = 0; k < kIdxBalanced / 64; k++)
-            if (qi >> 6 == k) len = __builtin_amdgcn_readlane(lens[k], qi & 63);
-        const int from = (max(len, 0) + kIdxTile - 1) / kIdxTile * kIdxTile;
+        const int from = (s_len[qi] + kIdxTile - 1) / kIdxTile * kIdxTile;
         for (int p = from + threadIdx.x; p < max_seq; p += blockDim.x) scores[(size_t)qi * max_seq + p] = -INFINITY;
     }
 }
@@ -501,13 +500,15 @@ static int device_cu_count() {
     return n;
 }
 
-// resident workgroups of the scoring kernel per CU (its register use sets it)
-template <int HT, bool P2>
+// resident workgroups of the scoring kernel per CU (its register use sets it, so
+// each form has its own: sized by the other's, equal runs at 16 and 32 heads ran
+// a second round of a third of the workgroups, 72.9 -> 78.9 us at Q=64 of 32768)
+template <int HT, bool P2, bool EVEN>
 static int scores_blocks_per_cu() {
     static std::atomic<int> cache{0};
     int b = cache.load(std::memory_order_relaxed);
     if (b <= 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, indexer_scores_kernel<HT, P2, false>, 256, 0) != hipSuccess || b <= 0)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, indexer_scores_kernel<HT, P2, EVEN>, 256, 0) != hipSuccess || b <= 0)
             b = 1;
         cache.store(b, std::memory_order_relaxed);
     }
@@ -515,11 +516,14 @@ static int scores_blocks_per_cu() {
 }
 
 // Workgroups per query of the scoring kernel, 0 for equal runs over all
-// queries' live tiles.  Equal runs begin with a load of every length, one
-// round trip more (1 us), so they are taken where a workgroup has at least 8
-// tiles (Q=64, 32768 positions, ragged: 83.8 -> 78.5 us with the selection,
-// equal lengths 89.8 -> 89.4; but Q=64, 8192 positions 36.0 -> 37.6), or 4
-// where whole parts do not fit the device at once (Q=50, 16384: 54.0 -> 48.9).
+// queries' live tiles; target: the workgroups of the other form that the device
+// holds at once.  Equal runs begin with a load of every length, one round trip
+// more (1 us), so they are taken where a workgroup has at least 8 tiles, or 4
+// where whole parts do not fit the device at once.  With the selection, us, lengths
+// drawn from [half, full] / all full, parts -> equal runs: Q=64 of 32768
+// positions 67.5 -> 64.1 / 73.5 -> 73.4 (32 heads), 73.9 -> 67.1 / 79.2 -> 79.0 (64);
+// Q=40 of 32768 63.6 -> 58.7 / 68.8 -> 66.3 (32 heads); Q=50 of 16384 56.1 -> 52.5 /
+// 57.8 -> 55.8 (64); but, not taken, Q=50 of 16384 all full 51.6 -> 53.5 (32).
 static int idx_parts_per_query(int Q, int ntile, long target) {
     const int parts = (int)std::max(1L, std::min((long)ntile, (target + Q - 1) / Q));
     const long tiles = (long)Q * ntile;
@@ -559,9 +563,10 @@ int launch_dsa_indexer(const uint8_t* qc, const float* qs, const float* hw, cons
     // the grid is the workgroups the device holds at once
 #define AMDMOE_IDX_LAUNCH2(HT, P2)                                                                      \
     do {                                                                                               \
-        const long target = (long)scores_blocks_per_cu<HT, P2>() * device_cu_count();                 \
-        const int nparts = idx_parts_per_query(Q, ntile, target);                                      \
-        const long grid = nparts ? (long)Q * nparts : std::min(target, (long)Q * ntile);               \
+        const long cus = device_cu_count();                                                            \
+        const int nparts = idx_parts_per_query(Q, ntile, scores_blocks_per_cu<HT, P2, false>() * cus); \
+        const long grid = nparts ? (long)Q * nparts                                                    \
+                                 : std::min(scores_blocks_per_cu<HT, P2, true>() * cus, (long)Q * ntile); \
         auto kern = nparts ? indexer_scores_kernel<HT, P2, false> : indexer_scores_kernel<HT, P2, true>; \
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, st, qc, qs, hw, kc, kb, ks,        \
                            page_table, seq_len, Q, page, shift, pages_per_seq, max_seq, ntile, nparts, \

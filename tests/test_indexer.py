@@ -295,7 +295,8 @@ def test_gpu_indexer_seq_len_past_page_table_capacity(amd, orc):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("Q,Hi,max_seq,page,topk", [(50, 16, 16384, 64, 64), (128, 16, 16384, 48, 32), (256, 16, 8192, 32, 16)])
+@pytest.mark.parametrize("Q,Hi,max_seq,page,topk", [(50, 16, 16384, 64, 64), (128, 16, 16384, 48, 32), (256, 16, 8192, 32, 16),
+                                                       (64, 32, 32768, 64, 64), (40, 32, 32768, 48, 32), (50, 64, 16384, 64, 32)])
 def test_gpu_indexer_equal_runs(amd, orc, Q, Hi, max_seq, page, topk):
     """Queries of very different lengths (empty, one position, tile edges, the
     full row) over the scoring kernel's equal runs, which then start and end
