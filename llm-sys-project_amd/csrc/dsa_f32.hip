@@ -25,8 +25,9 @@
 //       accumulating in the output rows; no scratch
 // The fold is the same sequence of operations in both, and a chunk depends
 // on the query's valid indices alone, so a row's result is bit-identical
-// whatever the batch around it, whichever kernel runs, and with or without
-// the invalid indices written out.
+// whatever the batch around it, whichever of the two runs, and with or without
+// the invalid indices written out (within one S: the smallest calls, by Dc, Dp
+// and S alone, run f32_small_kernel).
 //
 // What bounds it: at Q=8 H=16 Dc=512 Dp=64 S=1024 the call needs 24 MB
 // (5 us) and 0.29 GFLOP; it takes 19.5 us, two launches (16 + 4) of a few
@@ -504,7 +505,56 @@ __global__ __launch_bounds__(512) void f32_loop_kernel(DsaF32Args a) {
     }
 }
 
+// The smallest calls: a wave per (query, head), lane s with position s runs the
+// reference's sequential dots, lanes own output columns; every sum in the
+// reference's order.  One lane's chain of Dc + Dp products bounds it; the
+// kernels above take 9 us and more however small the call (512 threads, six
+// barriers), this one 4.6 at Q=1 H=1 Dc=32 Dp=4 S=1.
+__global__ __launch_bounds__(64) void f32_small_kernel(DsaF32Args a) {
+    __shared__ float s_p[64];
+    __shared__ int s_row[64];
+    const int qh = blockIdx.x, qi = qh / a.H, lane = threadIdx.x;
+    const int r = lane < a.S ? a.idx[(size_t)qi * a.S + lane] : -1;
+    const bool ok = r >= 0 && r < a.N;
+    float p = -INFINITY;
+    if (ok) {
+        const float *qn = a.qn + (size_t)qh * a.Dc, *qp = a.qp + (size_t)qh * a.Dp;
+        const float *kc = a.kc + (size_t)r * a.Dc, *kp = a.kp + (size_t)r * a.Dp;
+        float sc = 0.0f, sp = 0.0f;
+        for (int d = 0; d < a.Dc; d++) sc = mac_rn(sc, qn[d], kc[d]);
+        for (int d = 0; d < a.Dp; d++) sp = mac_rn(sp, qp[d], kp[d]);
+        p = mul_rn(add_rn(sc, sp), 1.0f / sqrtf((float)(a.Dc + a.Dp)));
+    }
+    const float mx = wave_max(p);
+    float* out = a.out + (size_t)qh * a.Dc;
+    if (mx == -INFINITY) {  // no score above -inf
+        for (int d = lane; d < a.Dc; d += 64) out[d] = 0.0f;
+        return;
+    }
+    p = expf(p - mx);
+    float tot = 0.0f;
+    for (int s = 0; s < a.S; s++) tot = add_rn(tot, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), s)));
+    s_p[lane] = __fdiv_rn(p, tot);
+    s_row[lane] = ok ? r : -1;
+    __syncthreads();
+    for (int d = lane; d < a.Dc; d += 64) {
+        float acc = 0.0f;
+        for (int s = 0; s < a.S; s++)
+            if (s_row[s] >= 0) acc = mac_rn(acc, s_p[s], a.v[(size_t)s_row[s] * a.Dc + d]);
+        out[d] = acc;
+    }
+}
+
 // ---------------------------------------------------------------- launch
+// Where f32_small_kernel is the faster one, from its time in ns: 2300 + 60 per
+// column + 170 (from 77 columns 2.2 per column) per position, against 9200 to
+// 10700 of the other kernel.  Measured at Dc + Dp = 36 / 80 / 160 / 576, S = 1 .. 64,
+// 1 to 1024 rows: 36 columns S=16 7.0 and 9.2 us, S=32 9.7 and 10.6, S=64 15.0 and
+// 10.9; 80 columns S=16 9.8 and 10.2, S=32 12.8 and 10.6; 160 columns S=1 11.9 and 10.6.
+static bool f32_small(int Dc, int Dp, int S) {
+    const long D = (long)Dc + Dp;
+    return S <= 64 && 600 * D + S * std::max(1700L, 22 * D) <= 77500;
+}
 // The split form runs where a workgroup per (query, 16 heads) leaves CUs
 // idle: fewer than 256 of them, and rows of more than one chunk.
 static long f32_head_tiles(int Q, int H) { return (long)Q * ((H + 15) / 16); }
@@ -556,6 +606,12 @@ int launch_dsa_f32(const float* qn, const float* qp, const float* kc, const floa
     DsaF32Args a{};
     a.qn = qn, a.qp = qp, a.kc = kc, a.kp = kp, a.v = v, a.idx = idx, a.out = out;
     a.H = H, a.Dc = Dc, a.Dp = Dp, a.S = S, a.N = N;
+    if (f32_small(Dc, Dp, S)) {
+        AMDMOE_CHECK_ARG((long)Q * H < (1L << 31), "dsa_forward: grid too large");
+        hipLaunchKernelGGL(f32_small_kernel, dim3((unsigned)((long)Q * H)), dim3(64), 0, st, a);
+        AMDMOE_LAUNCH_CHECK();
+        return AMDMOE_OK;
+    }
     // 16-byte loads: whole rows of 16 bytes at aligned bases (Dp = 0 reads no q_pe / K_p)
     auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool vec = Dc % 4 == 0 && Dp % 4 == 0 && al(qn) && al(kc) && al(v) && al(out) &&

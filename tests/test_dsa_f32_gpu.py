@@ -29,6 +29,9 @@ def _run(amd, t, shape):
 
 SHAPES = [
     (1, 1, 1, 0, 1, 1),          # the smallest call
+    (3, 2, 1, 0, 45, 64), (3, 2, 1, 0, 46, 64),    # a lane per position up to here, chunks from here
+    (2, 3, 30, 6, 32, 64), (2, 3, 30, 6, 33, 64), (3, 2, 64, 16, 16, 64), (3, 2, 64, 16, 17, 64),
+    (2, 2, 120, 4, 1, 8), (2, 2, 124, 8, 1, 8), (5, 40, 32, 4, 8, 64),
     (3, 5, 30, 6, 15, 40),       # unaligned rows, one partial tile
     (2, 16, 64, 16, 128, 300),   # the largest single chunk
     (2, 17, 100, 12, 129, 300),  # two head tiles, the first two-chunk row
@@ -172,6 +175,25 @@ def test_dsa_f32_many_streams(amd, n):
         assert torch.equal(out.cpu(), ref)
     for p in raw:
         assert lib.hipStreamDestroy(p) == 0
+
+
+@pytest.mark.parametrize("S", [6, 60])
+def test_dsa_f32_small_non_finite(amd, S):
+    """The same rules in the kernel of the smallest calls and in the next one."""
+    shape = (4, 2, 32, 4, S, 256)
+    a = list(_inputs(*shape, seed=6))
+    a[5][:] = np.arange(S) + 64 * np.arange(4)[:, None]
+    a[2][:, 0] = np.abs(a[2][:, 0]) + 0.1
+    a[2][2, 1] = np.nan       # one NaN score in query 0
+    a[0][1, 0, 0] = np.inf    # every score of a head
+    a[0][2, 1, 0] = -np.inf
+    a[5][3, S - 2:] = [-1, 256]
+    a[4][64 * 3 + S - 2:] = np.inf
+    out = _run(amd, [torch.from_numpy(x).cuda() for x in a], shape).cpu()
+    assert torch.isnan(out[0]).all()
+    assert torch.isnan(out[1, 0]).all() and torch.isfinite(out[1, 1]).all()
+    assert torch.isfinite(out[2, 0]).all() and (out[2, 1] == 0).all()
+    assert torch.isfinite(out[3]).all()
 
 
 def test_dsa_f32_non_finite(amd):
