@@ -636,7 +636,7 @@ __device__ __forceinline__ void route_exact_lds_body(const XT* __restrict__ x, c
     constexpr int PE = lane_pitch(E);
     s_logit[lt * PE + e] = sum;
     const int n = min(L::TPB, T - t0);
-    if (K <= 4) {
+    if (K <= 4 && n > 1) {  // (one token: the wave form, 0.6 us less at E=16)
         lane_route_tokens(s_logit, s_logit + L::TPB * PE, n, E, K, t0, idx, wts);
         return;
     }
@@ -966,6 +966,21 @@ __global__ __launch_bounds__(256) void route_topk_block_kernel(const float* __re
 }
 
 // ---------------------------------------------------------------- launch
+// Does route_exact_tile_kernel take less time than route_exact_kernel (tpb
+// tokens a block)?  Both in ns, fitted to 2250 calls (T = 1 .. 8192, E = 1 .. 32,
+// D = 7 .. 7168, x fp32 and bf16); the rule picks the faster one within 4% in all
+// but 20.  A lane's chain takes 6.5 a product from its own registers as long as
+// the wave loads few rows, more with each, 55 unaligned, and 850 and more per
+// token to route after the first; by tiles it takes 6.7 and 0.15 more per staged
+// row.  One token: D=4096 E=32 34 us, 56 by tiles; E=6 30 and 41.  16 tokens: D=4096
+// E=32 77 and 57, E=6 75 and 42, E=1 37 and 71.
+static bool route_by_tiles(int T, int E, int D, int tpb, bool vec, bool bf16) {
+    const int nt = std::min(T, tpb), lanes = nt * E, rows = 64 / E + E;
+    const int per = !vec ? 5500 : (bf16 ? 850 : (lanes <= 32 ? 650 : 860)) + 11 * std::max(0, lanes - 64);
+    const long exact = 4000 + (bf16 && vec ? 1000 : 0) + (E > 16 ? 1360 : 850) * ((nt + 1) / 2 - 1) + 30 * E + (long)D * per / 100;
+    const long tiles = 4300 + 55 * E + (long)D * (670 + 15 * rows) / 100;
+    return tiles < exact;
+}
 template <typename XT, typename GT>
 int launch_route_exact(const XT* x, const GT* wg, const float* bias, int T, int E, int K, int D,
                        int* idx, float* wts, hipStream_t st) {
@@ -995,7 +1010,7 @@ int launch_route_exact(const XT* x, const GT* wg, const float* bias, int T, int 
         }
         if (rc != -1) return rc;
     }
-    if (lane_route_supported(E, K)) {
+    if (lane_route_supported(E, K) && route_by_tiles(T, E, D, tpb, vec, sizeof(XT) == 2)) {
         const int tpb_l = 64 / E, rows = tpb_l + E, cs = tile_shift(rows, D);
         const size_t need = ((size_t)rows * ((1 << cs) + 4) + (size_t)tpb_l * (lane_pitch(E) + 1)) * 4;  // <= 50.2 KB
         const bool vec4 = D % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)wg & 15) == 0;

@@ -13,6 +13,8 @@ SHAPES = [  # T, E, K, D
     (4, 16, 4, 1000), (7, 31, 4, 129), (2, 32, 2, 1028), (33, 2, 2, 512), (40, 8, 2, 512),
     (40, 8, 4, 256), (9, 16, 3, 768),
     (6, 33, 4, 200), (6, 8, 5, 100),  # one past: the wave forms
+    (70, 31, 4, 129), (33, 32, 2, 1028), (45, 7, 3, 2049), (130, 1, 1, 5), (200, 24, 4, 36), (129, 5, 1, 261),
+    (1, 32, 2, 4096), (1, 6, 4, 1000), (2, 16, 4, 512), (1, 16, 2, 1024),  # a token or two
 ]
 
 
