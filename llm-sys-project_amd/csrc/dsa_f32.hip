@@ -63,7 +63,7 @@ struct DsaF32Args {
     int H, Dc, Dp, S;
     long N;
     int q0;            // split: the first query of this launch
-    int nc;            // split: chunk slots per (query, head tile)
+    int nc;            // split: chunk slots per (query, head tile); loop: whether O is in LDS
     float* part_o;     // [query - q0][head tile][chunk][16][Dc]
     float2* part_ml;   // [query - q0][head tile][chunk][16]; l < 0: no such chunk
 };
@@ -91,7 +91,7 @@ __device__ __forceinline__ f32x4 row4(const float* __restrict__ row, int k, int 
 // read 64 banks
 constexpr int kPPitch = kF32Max + 4, kSPitch = 68;
 struct DsaF32Lds {
-    int rows[kF32Max];                       // cache rows of the chunk
+    int rows[2][kF32Max];                    // cache rows of the chunk (loop: and of the next)
     float p[16 * kPPitch];                   // scores, then probabilities: [head][token]
     float part[kF32Waves * 16 * kSPitch];    // column parts of S^T, then token parts of O^T
     float m[16], l[16];
@@ -99,21 +99,22 @@ struct DsaF32Lds {
 };
 
 // The cache rows of valid positions [c0, c0 + cap) of a query, in order,
-// into L.rows; returns the query's number of valid positions.  Wave w counts
+// into rows; returns the query's number of valid positions.  Wave w counts
 // the indices of its eighth of the list, then places those of the window.
 // FIRST: n is not known yet; c0 is a chunk number and cap its chunk's length.
 // Each wave's first kKeep * 64 indices stay in registers between the two
 // passes (all of them up to S = 2048: one round trip instead of two).
-// The cursor is a wave's first group of 64 indices not placed in full and the
-// number of valid positions before it: the next window goes on there, so
-// walking all windows in turn reads the list once (read from the start for
-// every chunk, Q=260 H=16 Dc=64 S=32768 took 5084 us, now 3055).
+// The cursor is a wave's first group of 64 indices not placed in full, the
+// number of valid positions before it, and its indices, loaded ahead: the next
+// window goes on there, so walking all windows in turn reads the list once (read
+// from the start for every chunk, Q=260 H=16 Dc=64 S=32768 took 5084 us, now 2811).  The
+// caller's barrier follows.
 struct F32Cursor {
-    int s, base;
+    int s, base, r;
 };
 template <bool FIRST>
-__device__ __forceinline__ int f32_rows(const DsaF32Args& a, DsaF32Lds& L, const int* __restrict__ ir,
-                                        int n, int c0, int cap, F32Cursor& cur) {
+__device__ __forceinline__ int f32_rows(const DsaF32Args& a, DsaF32Lds& L, int* __restrict__ rows,
+                                        const int* __restrict__ ir, int n, int c0, int cap, F32Cursor& cur) {
     constexpr int kKeep = 4;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -123,15 +124,17 @@ __device__ __forceinline__ int f32_rows(const DsaF32Args& a, DsaF32Lds& L, const
         const int r = s < s1 ? ir[s] : -1;
         return r >= 0 && r < a.N ? r : -1;
     };
-    int s, base;
-    auto place = [&](int r) __attribute__((always_inline)) {  // the group at s
+    // the group at s, base valid positions before it; the next one is r2
+    int s = cur.s, base = cur.base;
+    auto place = [&](int r, int r2) __attribute__((always_inline)) {
         const unsigned long long mk = __ballot(r >= 0);
         const int at = base + __popcll(mk & ((1ull << lane) - 1)) - c0;
-        if (r >= 0 && at >= 0 && at < cap) L.rows[at] = r;
+        if (r >= 0 && at >= 0 && at < cap) rows[at] = r;
         base += __popcll(mk);
         s += 64;
-        if (base <= c0 + cap) cur = {s, base};
+        if (base <= c0 + cap) cur = {s, base, r2};
     };
+    int r = cur.r;
     if constexpr (FIRST) {
         int keep[kKeep];
 #pragma unroll
@@ -149,18 +152,17 @@ __device__ __forceinline__ int f32_rows(const DsaF32Args& a, DsaF32Lds& L, const
         s = s0;
         base = 0;
         for (int w = 0; w < wave; w++) base += L.cnt[w];
-        cur = {s, base};
-        if (base + c > c0) {  // (a wave whose indices all lie before the window places none)
+        cur = {s, base, keep[0]};
+        if (base + c <= c0) return n;  // (a wave whose indices all lie before the window places none)
+        r = index(s0 + 64 * kKeep + lane);
 #pragma unroll
-            for (int k = 0; k < kKeep; k++) place(keep[k]);
-            while (s < s1 && base < c0 + cap) place(index(s + lane));
-        }
-    } else {
-        s = cur.s;
-        base = cur.base;
-        while (s < s1 && base < c0 + cap) place(index(s + lane));
+        for (int k = 0; k < kKeep; k++) place(keep[k], k + 1 < kKeep ? keep[k + 1] : r);
     }
-    lds_barrier();
+    while (s < s1 && base < c0 + cap) {
+        const int r2 = index(s + 64 + lane);
+        place(r, r2);
+        r = r2;
+    }
     return n;
 }
 
@@ -182,24 +184,24 @@ __device__ __forceinline__ F32Pv f32_pv_split(int Dc, int len, int wave) {
 }
 constexpr int kPvB = 8;  // token groups whose V loads are in flight together
 template <bool VEC>
-__device__ __forceinline__ void f32_pv_load(const DsaF32Args& a, const DsaF32Lds& L, const F32Pv& w, int b,
+__device__ __forceinline__ void f32_pv_load(const DsaF32Args& a, const int* rows, const F32Pv& w, int b,
                                             int q, int len, f32x4 (&vv)[kPvB]) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < kPvB; j++) {
         const int tok = 4 * (q + j) + (lane >> 4);
         const bool ok = q + j < w.qb && tok < len;
-        const long row = L.rows[ok ? tok : 0];
+        const long row = rows[ok ? tok : 0];
         vv[j] = row4<VEC>(a.v + row * a.Dc, 64 * b + 4 * (lane & 15), a.Dc, ok && b < w.nb);
     }
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// (m, l) of a chunk of len (1 .. kF32Max) of the query's n positions, its rows
-// in L.rows: leaves p = expf(s - m) 2^-k in L.p, zero past len.  The first V loads
+// (m, l) of a chunk of len (1 .. kF32Max) of the query's n positions, its
+// rows in rows: leaves p = expf(s - m) 2^-k in L.p, zero past len.  The first V loads
 // of f32_pv go out (into vv) once the K loads have, under the softmax.
 template <bool VEC>
-__device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, int qi, int h0, int n, int len,
+__device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, const int* rows, int qi, int h0, int n, int len,
                                            float scale, f32x4 (&vv)[kPvB]) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -217,34 +219,39 @@ __device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, in
     for (int t = wave >> ks; t < nt; t += kF32Waves >> ks) {
         const int tok = 16 * t + c;
         const bool tok_ok = tok < len;
-        const long row = L.rows[tok_ok ? tok : 0];
+        const long row = rows[tok_ok ? tok : 0];
         const float* kc = a.kc + row * a.Dc;
         const float* kq = a.kp + row * a.Dp;
         f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        constexpr int kB = VEC ? 9 : 4;  // steps whose loads are in flight together
-        for (int s = sa; s < sb; s += kB) {
-            f32x4 kv[kB], qv[kB];
+        auto steps = [&](auto bc) __attribute__((always_inline)) {
+            constexpr int kB = decltype(bc)::value;  // steps whose loads are in flight together
+            for (int s = sa; s < sb; s += kB) {
+                f32x4 kv[kB], qv[kB];
 #pragma unroll
-            for (int j = 0; j < kB; j++) {
-                const bool live = s + j < sb;                    // uniform
-                const int st = live ? s + j : sa;
-                const bool first = st < nsc;                     // uniform
-                const int k = 16 * (first ? st : st - nsc) + 4 * g;
-                kv[j] = row4<VEC>(first ? kc : kq, k, first ? a.Dc : a.Dp, tok_ok && live);
-                qv[j] = row4<VEC>(first ? qn : qp, k, first ? a.Dc : a.Dp, hok && live);
+                for (int j = 0; j < kB; j++) {
+                    const bool live = s + j < sb;                // uniform
+                    const int st = live ? s + j : sa;
+                    const bool first = st < nsc;                 // uniform
+                    const int k = 16 * (first ? st : st - nsc) + 4 * g;
+                    kv[j] = row4<VEC>(first ? kc : kq, k, first ? a.Dc : a.Dp, tok_ok && live);
+                    qv[j] = row4<VEC>(first ? qn : qp, k, first ? a.Dc : a.Dp, hok && live);
+                }
+#pragma unroll
+                for (int j = 0; j < kB; j++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[i & 1] = mfma_f32(kv[j][i], qv[j][i], acc[i & 1]);
             }
-#pragma unroll
-            for (int j = 0; j < kB; j++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) acc[i & 1] = mfma_f32(kv[j][i], qv[j][i], acc[i & 1]);
-        }
+        };
+        // (a batch loads all of its steps, live or not)
+        if (VEC && per <= 3) steps(std::integral_constant<int, 3>());
+        else steps(std::integral_constant<int, VEC ? 9 : 4>());
         // lane: head c, tokens 16t + 4g + i; kp > 1: at most 4 tiles
         float* dst = kp == 1 ? L.p + c * kPPitch : L.part + (part * 16 + c) * kSPitch;
         *(f32x4*)(dst + 16 * t + 4 * g) = acc[0] + acc[1];
     }
     {
         const F32Pv w = f32_pv_split(a.Dc, len, wave);
-        f32_pv_load<VEC>(a, L, w, w.b, w.qa, len, vv);
+        f32_pv_load<VEC>(a, rows, w, w.b, w.qa, len, vv);
     }
     lds_barrier();
     // half a wave per head: lane j takes tokens j, j + 32, ...
@@ -279,7 +286,7 @@ __device__ __forceinline__ void f32_scores(const DsaF32Args& a, DsaF32Lds& L, in
 
 // O of the chunk, 64 dims at a time: store(head, dim, 4 values).
 template <bool VEC, typename Store>
-__device__ __forceinline__ void f32_pv(const DsaF32Args& a, DsaF32Lds& L, int len, f32x4 (&vv)[kPvB],
+__device__ __forceinline__ void f32_pv(const DsaF32Args& a, DsaF32Lds& L, const int* rows, int len, f32x4 (&vv)[kPvB],
                                        const Store& store) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -291,7 +298,7 @@ __device__ __forceinline__ void f32_pv(const DsaF32Args& a, DsaF32Lds& L, int le
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
         for (int q = w.qa; q < w.qb && b < nb; q += kPvB) {
-            if (q > w.qa || b > w.b) f32_pv_load<VEC>(a, L, w, b, q, len, vv);
+            if (q > w.qa || b > w.b) f32_pv_load<VEC>(a, rows, w, b, q, len, vv);
 #pragma unroll
             for (int j = 0; j < kPvB; j++) {
                 const int tok = 4 * (q + j) + g;
@@ -301,18 +308,18 @@ __device__ __forceinline__ void f32_pv(const DsaF32Args& a, DsaF32Lds& L, int le
             }
         }
         // acc[i][j], lane (head c, group g): dim 64b + 16g + 4j + i
-        if (tp > 1) {  // (then there is one round)
+        if (tp > 1) {  // (then there is one round; parts at kSPitch: at 64 all heads' stores share their banks)
             lds_barrier();
             if (b < nb)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    *(f32x4*)(L.part + wave * 1024 + c * 64 + 16 * g + 4 * j) =
+                    *(f32x4*)(L.part + (wave * 16 + c) * kSPitch + 16 * g + 4 * j) =
                         (f32x4){acc[0][j], acc[1][j], acc[2][j], acc[3][j]};
             lds_barrier();
             for (int e = tid; e < nb * 256; e += 64 * kF32Waves) {  // 4 dims of a head
                 const int bb = e >> 8, hd = (e >> 4) & 15, dd = 4 * (e & 15);
                 f32x4 o = {0.f, 0.f, 0.f, 0.f};
-                for (int k = 0; k < tp; k++) o += *(const f32x4*)(L.part + (bb * tp + k) * 1024 + hd * 64 + dd);
+                for (int k = 0; k < tp; k++) o += *(const f32x4*)(L.part + ((bb * tp + k) * 16 + hd) * kSPitch + dd);
                 store(hd, 64 * bb + dd, o);
             }
         } else if (b < nb) {
@@ -360,19 +367,20 @@ __global__ __launch_bounds__(512) void f32_split_kernel(DsaF32Args a) {
     const int ht = (a.H + 15) >> 4;
     const int sp = blockIdx.x % a.nc, qt = blockIdx.x / a.nc;
     const int qi = a.q0 + qt / ht, h0 = 16 * (qt % ht);
-    F32Cursor cur;
-    const int n = f32_rows<true>(a, L, a.idx + (size_t)qi * a.S, 0, sp, 0, cur);
+    F32Cursor cur = {0, 0, -1};
+    const int n = f32_rows<true>(a, L, L.rows[0], a.idx + (size_t)qi * a.S, 0, sp, 0, cur);
     const int chunk = f32_chunk(n), c0 = sp * chunk;
     const size_t slot = (size_t)blockIdx.x * 16;
     if (c0 >= n) {
         if (threadIdx.x < 16) a.part_ml[slot + threadIdx.x] = make_float2(-INFINITY, -1.0f);
         return;
     }
+    lds_barrier();
     const int len = min(chunk, n - c0);
     f32x4 vv[kPvB];
-    f32_scores<VEC>(a, L, qi, h0, n, len, 1.0f / sqrtf((float)(a.Dc + a.Dp)), vv);
+    f32_scores<VEC>(a, L, L.rows[0], qi, h0, n, len, 1.0f / sqrtf((float)(a.Dc + a.Dp)), vv);
     if (threadIdx.x < 16) a.part_ml[slot + threadIdx.x] = make_float2(L.m[threadIdx.x], L.l[threadIdx.x]);
-    f32_pv<VEC>(a, L, len, vv, [&](int hd, int d, f32x4 o) __attribute__((always_inline)) {
+    f32_pv<VEC>(a, L, L.rows[0], len, vv, [&](int hd, int d, f32x4 o) __attribute__((always_inline)) {
         if (h0 + hd < a.H) store4<VEC>(a.part_o + (slot + hd) * a.Dc, d, a.Dc, o);
     });
 }
@@ -451,56 +459,65 @@ __global__ __launch_bounds__(64) void f32_merge_kernel(DsaF32Args a) {
     store4<VEC>(a.out + ((size_t)(a.q0 + ql) * a.H + hd) * a.Dc, d, a.Dc, r);
 }
 
+// The same fold by one workgroup: a thread has the same dims of the same head in
+// every chunk, so it keeps that head's (m, l) and O, in LDS where there is room
+// (nc = 1: up to 320 columns for two workgroups on a CU, 512 for one), else in
+// the output rows.
+// The next chunk's rows are placed before the barrier that ends a chunk, from
+// indices loaded a chunk earlier.  A chunk is a chain of latencies: Q=4 H=8 Dc=32
+// S=1024 (32 chunks) in one launch took 278 us with O in the output rows, the fold
+// between two barriers of its own and bank conflicts in the token parts (21000
+// cycles a chunk, 4300 of them those stores, 6600 rows and scores), 178 so.
+constexpr int kLoopDc2 = 320, kLoopDc1 = 512;
+__host__ __device__ inline int f32_loop_pitch(int Dc) { return ((Dc + 63) & ~63) + 4; }
 template <bool VEC>
-__global__ __launch_bounds__(512) void f32_loop_kernel(DsaF32Args a) {
+__global__ __launch_bounds__(512, 4) void f32_loop_kernel(DsaF32Args a) {
     __shared__ DsaF32Lds L;
-    __shared__ float s_m[16], s_l[16];
-    __shared__ F32Fold s_f[16];
+    extern __shared__ __attribute__((aligned(16))) float s_o[];  // [head][f32_loop_pitch(Dc)]
     const int ht = (a.H + 15) >> 4;
     const int qi = blockIdx.x / ht, h0 = 16 * (blockIdx.x % ht);
     const int tid = threadIdx.x;
     const int* ir = a.idx + (size_t)qi * a.S;
     float* orow = a.out + ((size_t)qi * a.H + h0) * a.Dc;
     const float scale = 1.0f / sqrtf((float)(a.Dc + a.Dp));
-    if (tid < 16) s_m[tid] = -INFINITY, s_l[tid] = 0.0f;
-    F32Cursor cur;
-    const int n = f32_rows<true>(a, L, ir, 0, 0, 0, cur);
+    const bool lds_o = a.nc != 0;
+    const int pitch = f32_loop_pitch(a.Dc);
+    const int hd_own = a.Dc <= 256 ? (tid >> 4) & 15 : tid & 15;  // the head f32_pv gives this thread
+    float m = -INFINITY, l = 0.0f;                                // of that head
+    F32Cursor cur = {0, 0, -1};
+    const int n = f32_rows<true>(a, L, L.rows[0], ir, 0, 0, 0, cur);
     if (n == 0) {  // no valid index
         for (int i = tid; i < 16 * a.Dc; i += 512)
             if (h0 + i / a.Dc < a.H) orow[i] = 0.0f;
         return;
     }
     const int chunk = f32_chunk(n);
-    for (int c0 = 0; c0 < n; c0 += chunk) {
-        if (c0) {
-            lds_barrier();  // the last chunk's rows and probabilities have been read
-            f32_rows<false>(a, L, ir, n, c0, chunk, cur);
-        }
+    int buf = 0;
+    for (int c0 = 0; c0 < n; c0 += chunk, buf ^= 1) {
+        if (c0) f32_rows<false>(a, L, L.rows[buf], ir, n, c0, chunk, cur);
+        lds_barrier();  // the rows are there, the last chunk's probabilities have been read
         const int len = min(chunk, n - c0);
         f32x4 vv[kPvB];
-        f32_scores<VEC>(a, L, qi, h0, n, len, scale, vv);
-        if (tid < 16) {
-            float m = s_m[tid], l = s_l[tid];
-            s_f[tid] = f32_fold(m, l, L.m[tid], L.l[tid]);
-            s_m[tid] = m;
-            s_l[tid] = l;
-        }
-        lds_barrier();
+        f32_scores<VEC>(a, L, L.rows[buf], qi, h0, n, len, scale, vv);
+        const F32Fold f = f32_fold(m, l, L.m[hd_own], L.l[hd_own]);
+        const float inv = f32_inv(m, l);
         const bool last = c0 + chunk >= n;
-        // a thread stores the same dims in every chunk, so it reads back its own sums
-        f32_pv<VEC>(a, L, len, vv, [&](int hd, int d, f32x4 oj) __attribute__((always_inline)) {
+        f32_pv<VEC>(a, L, L.rows[buf], len, vv, [&](int hd, int d, f32x4 oj) __attribute__((always_inline)) {
             if (h0 + hd >= a.H) return;
             float* row = orow + (size_t)hd * a.Dc;
-            const F32Fold f = s_f[hd];
+            float* so = s_o + hd * pitch + d;
             f32x4 o = {0.f, 0.f, 0.f, 0.f};
-            if (c0) o = row4<VEC>(row, d, a.Dc, true);
-            const float m = s_m[hd], inv = f32_inv(m, s_l[hd]);
+            if (c0) {
+                if (lds_o) o = *(const f32x4*)so;
+                else o = row4<VEC>(row, d, a.Dc, true);
+            }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 o[i] = f32_fold_o(f, o[i], oj[i]);
                 if (last) o[i] = m == -INFINITY ? 0.0f : mul_rn(o[i], inv);
             }
-            store4<VEC>(row, d, a.Dc, o);
+            if (lds_o && !last) *(f32x4*)so = o;
+            else store4<VEC>(row, d, a.Dc, o);
         });
     }
 }
@@ -577,7 +594,11 @@ static int launch_f32(DsaF32Args a, int Q, void* scratch, size_t scratch_bytes, 
     const long tiles = f32_head_tiles(Q, a.H);
     if (!scratch) {
         AMDMOE_CHECK_ARG(tiles < (1L << 31), "dsa_forward: grid too large");
-        hipLaunchKernelGGL(f32_loop_kernel<VEC>, dim3((unsigned)tiles), dim3(512), 0, st, a);
+        a.nc = a.Dc <= (tiles <= 256 ? kLoopDc1 : kLoopDc2);
+        const int lds = a.nc ? 16 * f32_loop_pitch(a.Dc) * 4 : 0;
+        const int rc = ensure_dynamic_lds((const void*)f32_loop_kernel<VEC>, 16 * f32_loop_pitch(kLoopDc1) * 4);
+        if (rc != AMDMOE_OK) return rc;
+        hipLaunchKernelGGL(f32_loop_kernel<VEC>, dim3((unsigned)tiles), dim3(512), lds, st, a);
         AMDMOE_LAUNCH_CHECK();
         return AMDMOE_OK;
     }
