@@ -26,8 +26,8 @@
 // The fold is the same sequence of operations in both, and a chunk depends
 // on the query's valid indices alone, so a row's result is bit-identical
 // whatever the batch around it, whichever of the two runs, and with or without
-// the invalid indices written out (within one S: the smallest calls, by Dc, Dp
-// and S alone, run f32_small_kernel).
+// the invalid indices written out.  The smallest calls, and many rows of few
+// heads and columns, run f32_row_kernel instead (f32_by_rows).
 //
 // What bounds it: at Q=8 H=16 Dc=512 Dp=64 S=1024 the call needs 24 MB
 // (5 us) and 0.29 GFLOP; it takes 19.5 us, two launches (16 + 4) of a few
@@ -522,59 +522,96 @@ __global__ __launch_bounds__(512, 4) void f32_loop_kernel(DsaF32Args a) {
     }
 }
 
-// The smallest calls: a wave per (query, head), lane s with position s runs the
-// reference's sequential dots, lanes own output columns; every sum in the
-// reference's order.  One lane's chain of Dc + Dp products bounds it; the
-// kernels above take 9 us and more however small the call (512 threads, six
-// barriers), this one 4.6 at Q=1 H=1 Dc=32 Dp=4 S=1.
-__global__ __launch_bounds__(64) void f32_small_kernel(DsaF32Args a) {
-    __shared__ float s_p[64];
-    __shared__ int s_row[64];
+// A wave per (query, head), lane j with positions j, j + 64, ...: four sums over
+// the columns of its rows, then lanes own output columns.  For the smallest
+// calls, where the kernels above take 9 us however little there is to do (512
+// threads, six barriers), and for many rows of few heads and columns, where they
+// run whole chunks for one or two of a tile's 16 heads.
+template <bool VEC>
+__global__ __launch_bounds__(64) void f32_row_kernel(DsaF32Args a) {
+    extern __shared__ float s_p[];  // [S] scores, then probabilities
+    int* s_row = (int*)(s_p + a.S);
     const int qh = blockIdx.x, qi = qh / a.H, lane = threadIdx.x;
-    const int r = lane < a.S ? a.idx[(size_t)qi * a.S + lane] : -1;
-    const bool ok = r >= 0 && r < a.N;
-    float p = -INFINITY;
-    if (ok) {
-        const float *qn = a.qn + (size_t)qh * a.Dc, *qp = a.qp + (size_t)qh * a.Dp;
-        const float *kc = a.kc + (size_t)r * a.Dc, *kp = a.kp + (size_t)r * a.Dp;
-        float sc = 0.0f, sp = 0.0f;
-        for (int d = 0; d < a.Dc; d++) sc = mac_rn(sc, qn[d], kc[d]);
-        for (int d = 0; d < a.Dp; d++) sp = mac_rn(sp, qp[d], kp[d]);
-        p = mul_rn(add_rn(sc, sp), 1.0f / sqrtf((float)(a.Dc + a.Dp)));
+    const float *qn = a.qn + (size_t)qh * a.Dc, *qp = a.qp + (size_t)qh * a.Dp;
+    const int* ir = a.idx + (size_t)qi * a.S;
+    const float scale = 1.0f / sqrtf((float)(a.Dc + a.Dp));
+    float mx = -INFINITY;
+    for (int s = lane; s < a.S; s += 64) {
+        const int r = ir[s];
+        const bool ok = r >= 0 && r < a.N;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        auto dot = [&](const float* q, const float* k, int D) __attribute__((always_inline)) {
+#pragma unroll 4
+            for (int d = 0; d < D; d += 4) {
+                const f32x4 kv = row4<VEC>(k, d, D, true), qv = row4<VEC>(q, d, D, true);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] = fmaf(kv[i], qv[i], acc[i]);
+            }
+        };
+        float p = -INFINITY;
+        if (ok) {
+            dot(qn, a.kc + (size_t)r * a.Dc, a.Dc);
+            dot(qp, a.kp + (size_t)r * a.Dp, a.Dp);
+            p = ((acc[0] + acc[1]) + (acc[2] + acc[3])) * scale;
+        }
+        mx = fmaxf(mx, p);
+        s_p[s] = p;
+        s_row[s] = ok ? r : -1;
     }
-    const float mx = wave_max(p);
+    mx = wave_max(mx);
     float* out = a.out + (size_t)qh * a.Dc;
     if (mx == -INFINITY) {  // no score above -inf
         for (int d = lane; d < a.Dc; d += 64) out[d] = 0.0f;
         return;
     }
-    p = expf(p - mx);
     float tot = 0.0f;
-    for (int s = 0; s < a.S; s++) tot = add_rn(tot, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), s)));
-    s_p[lane] = __fdiv_rn(p, tot);
-    s_row[lane] = ok ? r : -1;
+    for (int s = lane; s < a.S; s += 64) tot += s_p[s] = expf(s_p[s] - mx);
+    tot = wave_sum(tot);
+    for (int s = lane; s < a.S; s += 64) s_p[s] = __fdiv_rn(s_p[s], tot);
     __syncthreads();
     for (int d = lane; d < a.Dc; d += 64) {
-        float acc = 0.0f;
-        for (int s = 0; s < a.S; s++)
-            if (s_row[s] >= 0) acc = mac_rn(acc, s_p[s], a.v[(size_t)s_row[s] * a.Dc + d]);
-        out[d] = acc;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+        for (int s = 0; s < a.S; s += 4) {
+            float v[4], p[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int t = min(s + i, a.S - 1), r = s_row[t];
+                const bool ok = s + i < a.S && r >= 0;
+                const float x = a.v[(size_t)max(r, 0) * a.Dc + d];
+                v[i] = ok ? x : 0.0f;
+                p[i] = ok ? s_p[t] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i] = fmaf(p[i], v[i], acc[i]);
+        }
+        out[d] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     }
 }
 
 // ---------------------------------------------------------------- launch
-// Where f32_small_kernel is the faster one, from its time in ns: 2300 + 60 per
-// column + 170 (from 77 columns 2.2 per column) per position, against 9200 to
-// 10700 of the other kernel.  Measured at Dc + Dp = 36 / 80 / 160 / 576, S = 1 .. 64,
-// 1 to 1024 rows: 36 columns S=16 7.0 and 9.2 us, S=32 9.7 and 10.6, S=64 15.0 and
-// 10.9; 80 columns S=16 9.8 and 10.2, S=32 12.8 and 10.6; 160 columns S=1 11.9 and 10.6.
-static bool f32_small(int Dc, int Dp, int S) {
-    const long D = (long)Dc + Dp;
-    return S <= 64 && 600 * D + S * std::max(1700L, 22 * D) <= 77500;
+static long f32_head_tiles(int Q, int H) { return (long)Q * ((H + 15) / 16); }
+// Is f32_row_kernel the faster one?  Both times in ns, fitted to 1000 calls (Q = 1
+// .. 2500, H = 1 .. 16, Dc = 8 .. 512, S = 1 .. 1024): a wave's chain over its
+// positions and their traffic, against one chunk (8 us, in rounds of 512
+// workgroups) or a full chip's walks (5.5 us per chunk, 7.6 with two workgroups
+// on a CU); a row of several chunks on few CUs is always split.  Tiles and rows,
+// us: Q=1 H=1 Dc=32 Dp=4 S=1 8.0 and 3.8, S=64 9.1 and 9.0; Dc=128 Dp=32 S=16 9.1 and
+// 7.2, S=32 9.2 and 9.9; Q=1000 H=1 Dc=32 S=1024 486 and 116; Q=1000 H=4 Dc=128 513
+// and 506; Q=256 H=16 Dc=64 185 and 253.  It depends on the shape alone, so eager
+// and captured calls agree.
+static bool f32_by_rows(int Q, int H, int Dc, int Dp, int S) {
+    const long tiles = f32_head_tiles(Q, H), rows = (long)Q * H, D = (long)Dc + Dp;
+    if (S > 2048 || (S > kF32One && tiles < 256)) return false;
+    const long rounds = (tiles + 511) / 512;
+    const float row = 3200.0f + 13.0f * D + (float)S * ((Dc + 63) / 64) * (82.0f + 0.042f * rows);
+    const float tile = S > kF32One      ? 4000.0f + (S + f32_chunk(S) - 1) / f32_chunk(S) * rounds * (tiles <= 256 ? 5500.0f : 7600.0f)
+                       : tiles <= 256 ? 8000.0f + 3.6f * D + 12.0f * S
+                                      : 4000.0f + rounds * (8000.0f + 30.0f * S);
+    return row < 0.95f * tile;
 }
 // The split form runs where a workgroup per (query, 16 heads) leaves CUs
 // idle: fewer than 256 of them, and rows of more than one chunk.
-static long f32_head_tiles(int Q, int H) { return (long)Q * ((H + 15) / 16); }
 static size_t f32_query_bytes(int H, int Dc, int S) {  // partials of one query
     const size_t slots = (size_t)((H + 15) / 16) * f32_max_chunks(S) * 16;
     return slots * Dc * 4 + slots * 8;
@@ -627,16 +664,17 @@ int launch_dsa_f32(const float* qn, const float* qp, const float* kc, const floa
     DsaF32Args a{};
     a.qn = qn, a.qp = qp, a.kc = kc, a.kp = kp, a.v = v, a.idx = idx, a.out = out;
     a.H = H, a.Dc = Dc, a.Dp = Dp, a.S = S, a.N = N;
-    if (f32_small(Dc, Dp, S)) {
-        AMDMOE_CHECK_ARG((long)Q * H < (1L << 31), "dsa_forward: grid too large");
-        hipLaunchKernelGGL(f32_small_kernel, dim3((unsigned)((long)Q * H)), dim3(64), 0, st, a);
-        AMDMOE_LAUNCH_CHECK();
-        return AMDMOE_OK;
-    }
     // 16-byte loads: whole rows of 16 bytes at aligned bases (Dp = 0 reads no q_pe / K_p)
     auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool vec = Dc % 4 == 0 && Dp % 4 == 0 && al(qn) && al(kc) && al(v) && al(out) &&
                      (Dp == 0 || (al(qp) && al(kp)));
+    if (f32_by_rows(Q, H, Dc, Dp, S)) {
+        AMDMOE_CHECK_ARG((long)Q * H < (1L << 31), "dsa_forward: grid too large");
+        auto kern = vec ? f32_row_kernel<true> : f32_row_kernel<false>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((long)Q * H)), dim3(64), 8 * (size_t)S, st, a);
+        AMDMOE_LAUNCH_CHECK();
+        return AMDMOE_OK;
+    }
     return vec ? launch_f32<true>(a, Q, scratch, scratch_bytes, st)
                : launch_f32<false>(a, Q, scratch, scratch_bytes, st);
 }

@@ -29,9 +29,9 @@ def _run(amd, t, shape):
 
 SHAPES = [
     (1, 1, 1, 0, 1, 1),          # the smallest call
-    (3, 2, 1, 0, 45, 64), (3, 2, 1, 0, 46, 64),    # a lane per position up to here, chunks from here
-    (2, 3, 30, 6, 32, 64), (2, 3, 30, 6, 33, 64), (3, 2, 64, 16, 16, 64), (3, 2, 64, 16, 17, 64),
-    (2, 2, 120, 4, 1, 8), (2, 2, 124, 8, 1, 8), (5, 40, 32, 4, 8, 64),
+    (3, 2, 1, 0, 45, 64), (2, 3, 30, 6, 33, 64), (3, 2, 64, 16, 17, 64), (2, 2, 120, 4, 1, 8),  # a wave per row
+    (5, 40, 32, 4, 8, 64), (2, 2, 320, 4, 3, 8), (3, 2, 1, 0, 70, 100), (3, 2, 64, 16, 60, 64),  # and chunks
+    (256, 1, 32, 8, 129, 256), (300, 2, 31, 5, 300, 512), (600, 1, 100, 20, 1025, 2048),  # many rows
     (3, 5, 30, 6, 15, 40),       # unaligned rows, one partial tile
     (2, 16, 64, 16, 128, 300),   # the largest single chunk
     (2, 17, 100, 12, 129, 300),  # two head tiles, the first two-chunk row
