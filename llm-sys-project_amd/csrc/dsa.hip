@@ -665,8 +665,8 @@ __global__ __launch_bounds__(64) void dsa_merge_f32_kernel(const float* __restri
 // the first tile (page table, q) and a slope, which rises where the
 // workgroups share the memory (32 heads, S=2048 Q=1: 59.5, S=600 on 256 CUs: 28.5).
 static float split_us(int hg, int n, float load) {
-    if (hg == 32 && n > 2 && n * kT32 <= SplitGeom<2, 2>::CHUNK) return 8.8f + (0.8f + 0.24f * load) * n;
-    if (hg == 32) return 7.0f + (n > 2 ? 1.5f : 1.2f) * n;
+    if (hg == 32 && n > 3 && n * kT32 <= SplitGeom<2, 2>::CHUNK) return 8.8f + (0.8f + 0.24f * load) * n;
+    if (hg == 32) return 7.3f + (n > 3 ? 1.5f : 1.3f) * n;
     if (hg == 64) return 8.3f + 1.58f * n;
     if (hg == 96) return 11.0f + 1.5f * n;
     return 8.4f + (1.8f + 0.5f * load) * n;
@@ -754,9 +754,10 @@ int launch_dsa_bf16_paged(const uint16_t* qn, const uint16_t* qp, const uint16_t
     AMDMOE_CHECK_ARG(grid < (1L << 31), "dsa_decode_bf16_paged: grid too large");
     float* part_ml = plan.bytes ? (float*)((uint8_t*)scratch + align_up((size_t)Q * ns * H * kDc * (hg == 128 ? 2 : 4), 256))
                                : nullptr;
-    // two token groups from three tiles on (S=64 Q=64 H=32: 9.1 us without, 10.0
-    // with), up to the positions its LDS has room for beside four stages
-    const bool pair = hg == 32 && chunk > 2 * kT32 && chunk <= SplitGeom<2, 2>::CHUNK;
+    // two token groups from four tiles on (Q=64 H=32, us without and with: S=64 9.8
+    // and 10.4, S=96 11.1 and 12.0, S=112 12.4 and 12.0, S=224 16.9 and 15.2), up to
+    // the positions its LDS has room for beside four stages
+    const bool pair = hg == 32 && chunk > 3 * kT32 && chunk <= SplitGeom<2, 2>::CHUNK;
     auto split = hg == 128  ? (wide ? dsa_split_wide_kernel : dsa_split_kernel)
                  : hg == 96 ? dsa_split96_kernel
                  : hg == 64 ? (wide ? dsa_split64_wide_kernel : dsa_split64_kernel)

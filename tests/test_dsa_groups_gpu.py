@@ -33,7 +33,7 @@ SHAPES = [
     (130, 96, 3072, 4096), (130, 96, 3073, 4096), (131, 96, 4096, 4096),  # 96-head groups: rounds of 1536 positions
     (1, 128, 2048, 4096), (3, 256, 65, 256), (64, 128, 64, 256), (1, 384, 4096, 8192),  # H a multiple of 128
     (1, 128, 4097, 8192),  # past the small groups' positions: 128 heads
-    (257, 32, 65, 128), (260, 32, 96, 128), (257, 32, 97, 128),  # two token groups: 3 and 4 tiles, a ragged one
+    (257, 32, 65, 128), (260, 32, 96, 128), (257, 32, 97, 128), (260, 32, 160, 192),  # two token groups from 4 tiles on
     (257, 32, 3072, 3072), (257, 32, 3073, 3136),  # their most positions, and past it
     (64, 96, 512, 1024), (32, 192, 512, 1024),
 ]
