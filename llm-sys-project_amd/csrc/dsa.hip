@@ -666,7 +666,7 @@ __global__ __launch_bounds__(64) void dsa_merge_f32_kernel(const float* __restri
 // workgroups share the memory (32 heads, S=2048 Q=1: 59.5, S=600 on 256 CUs: 28.5).
 static float split_us(int hg, int n, float load) {
     if (hg == 32 && n > 3 && n * kT32 <= SplitGeom<2, 2>::CHUNK) return 8.8f + (0.8f + 0.24f * load) * n;
-    if (hg == 32) return 7.3f + (n > 3 ? 1.5f : 1.3f) * n;
+    if (hg == 32) return 7.3f + (n > 3 ? 1.5f : 1.3f) * std::max(n, 2);  // (the first two tiles load together)
     if (hg == 64) return 8.3f + 1.58f * n;
     if (hg == 96) return 11.0f + 1.5f * n;
     return 8.4f + (1.8f + 0.5f * load) * n;
@@ -678,8 +678,8 @@ static float split_us(int hg, int n, float load) {
 // groups of 32, 64 or 96 heads (S <= 4096): any split that fits the CUs at
 // once, more than one only with scratch.  The cheapest by a model
 // fitted to measured calls (us): workgroups run in rounds of 256, a merge takes
-// 4 + 0.2 per split (0.5 in the 128-head merge, four splits a round trip) and
-// moves its partials at 8 MB per us (16 where they are bf16).
+// 3 + 0.1 per split and moves its partials at 5.3 MB per us (the 128-head
+// merge 4 + 0.5, four splits a round trip, and 16 MB per us of bf16).
 // So few queries take many splits of small groups (S=2000 Q=4 H=64: 61 us in one
 // split of 32 heads, 19 in 16; S=2048 Q=1 H=128: 48 us in 64 splits of 128 heads,
 // 17 so), short selections one split of small groups (S=64 Q=64 H=128: 20 ->
@@ -695,7 +695,7 @@ DsaPlan dsa_paged_plan(int Q, int H, int S, bool scratch) {
         const float rounds = (float)((wgs + 255) / 256), load = std::min(1.0f, wgs / 256.0f);
         float us = rounds * split_us(hg, (tiles + ns - 1) / ns, load);
         if (hg == 128) us += 4.0f + 0.5f * ns + 2.0f * ns * Q * H * (kDc * 2) / 16e6f;
-        else if (ns > 1) us += 4.0f + 0.2f * ns + 2.0f * ns * Q * H * (kDc * 4) / 8e6f;
+        else if (ns > 1) us += 3.0f + 0.1f * ns + 2.0f * ns * Q * H * (kDc * 4) / 5.3e6f;
         return us;
     };
     if (H % 128 == 0) {
