@@ -484,7 +484,7 @@ def traffic_summary(fetch_dir, write_dir, out_md, out_json, command,
         rows.append(f"| `{k}` | {fa[k]['FETCH_SIZE']:.4g} | {wa[k]['WRITE_SIZE']:.4g} | "
                     f"{(fb + wb) / 1e9:.3f} GB |")
     lines = [f"# {title}", "",
-             "Two counter runs and the summary (from the repository root on the GPU box):", "",
+             "Two counter runs and the summary (from the repository root, on an MI355X):", "",
              "```", command, "```", "",
              f"Calibration: `--calibrate-copy` runs one 1 GiB device-to-device copy first "
              f"(`{c}`, {fa[c]['dispatches']} dispatches).  Per dispatch FETCH_SIZE reads "
@@ -508,7 +508,7 @@ def stats_summary(csv_dir, out_md, title, command):
     files = glob.glob(os.path.join(csv_dir, "**", "*kernel_stats.csv"), recursive=True)
     if not files:
         raise SystemExit(f"no kernel_stats.csv under {csv_dir}")
-    lines = [f"# {title}", "", "Command (from the repository root on the GPU box):", "", "```",
+    lines = [f"# {title}", "", "Command (from the repository root, on an MI355X):", "", "```",
              command, "```", "",
              "Rows: this library's kernels (torch and rocprim kernels of the synthetic-data "
              "setup omitted).", "",
@@ -575,7 +575,7 @@ def pmc_summary(csv_dir, out_md, title, command):
         derived.append(("LDS conflict", lambda a: a["SQ_LDS_BANK_CONFLICT"] / max(a["SQ_ACTIVE_INST_LDS"], 1.0)))
     if {"TCC_HIT_sum", "TCC_MISS_sum"} <= have:
         derived.append(("L2 hit", lambda a: a["TCC_HIT_sum"] / max(a["TCC_HIT_sum"] + a["TCC_MISS_sum"], 1.0)))
-    lines = [f"# {title}", "", "Command (from the repository root on the GPU box):", "", "```",
+    lines = [f"# {title}", "", "Command (from the repository root, on an MI355X):", "", "```",
              command, "```", "",
              "Per kernel: each counter summed over its hardware instances per dispatch, averaged "
              "over the kernel's dispatches."]

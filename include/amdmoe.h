@@ -33,11 +33,11 @@
  *     on any streams and threads at once: their scratch is one buffer per
  *     stream (at most 256 of at most 64 MiB, 4 GiB together; the call that
  *     makes or grows one may wait for the device, and a call past these
- *     bounds allocates and frees in stream order).  A captured call uses none and takes a form
- *     without: the fp32 attention gives the same bits, slower (Q=8 H=16 Dc=512
+ *     bounds allocates and frees in stream order).  A captured call uses none
+ *     and takes a form without: the fp32 attention gives the same bits, slower (Q=8 H=16 Dc=512
  *     Dp=64 S=1024 290 us for 19); the decode rounds differently than the
  *     eager call, within its tolerance, and runs one split per query (Q=4 H=64
- *     S=2000 61 us for 19).  Synchronise a stream that was passed to these two
+ *     S=2000 65 us for 19).  Synchronise a stream that was passed to these two
  *     before destroying it: another stream may get its handle, and so its
  *     buffer.
  *   - bf16 tensors are passed as uint16_t (bfloat16 bit patterns), fp8 as

@@ -36,7 +36,9 @@ constexpr uint32_t kOobDsa = 0xFFFFF000u;
 constexpr long kMaxCacheBytes = 0xFFFFE000L;
 constexpr int kDc = 512, kDp = 64, kDt = 576;
 constexpr int kRowBytes = kDt * 2;               // 1152
-constexpr int kMaxS = 4096;  // selected positions per query where H is no multiple of 128
+// The most positions of one split of a group of 32, 64 or 96 heads, and so the
+// most selected positions per query where H is no multiple of 128.
+constexpr int kMaxS = 4096;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -73,7 +75,8 @@ typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
 // ring (each tile's loads go out two tiles ahead), filled by direct
 // global->LDS loads; each wave reads every tile once for S and once for V.
 // dsa_split96/64/32_kernel are the same body with 6, 4 and 2 waves, for groups
-// of that many heads: no skew between waves, so a 3-stage ring and room for the
+// of that many heads (of any H, a multiple of 128 too, where the plan below
+// finds them faster): no skew between waves, so a 3-stage ring and room for the
 // rows of 4096 positions.  A wave alone on its SIMD waits for LDS and for its
 // own softmax (1.5 us per tile for 0.45 of MFMAs), and with 32 heads half of
 // the SIMDs have none: dsa_split32x2_kernel gives every second tile to a second
@@ -135,7 +138,7 @@ static __device__ __align__(16) uint16_t g_dsa_zero_row[kDt];
 
 // WIDE: the cache is addressed with 64-bit per-lane pointers
 // (global_load_lds_dwordx4) instead of a buffer descriptor's 32-bit offsets.
-// The body is a device template behind two plain kernels (the host side
+// The body is a device template behind plain kernels (the host side
 // dropped the launch stub of a templated kernel instantiation using buffer
 // descriptors).
 //
@@ -602,7 +605,7 @@ __global__ __launch_bounds__(256) void dsa_merge_kernel(const uint16_t* __restri
     }
 }
 
-// The same for the fp32 partials of dsa_split96/64/32_kernel.  These calls are
+// The same for the fp32 partials of the small head groups' kernels.  These calls are
 // small (fewer than 256 head groups) and have up to a few dozen
 // splits, so a workgroup is one wave per (query, 16 heads, two dim tiles),
 // eight splits' loads in flight.

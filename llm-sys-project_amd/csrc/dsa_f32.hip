@@ -25,9 +25,10 @@
 //       accumulating in the output rows; no scratch
 // The fold is the same sequence of operations in both, and a chunk depends
 // on the query's valid indices alone, so a row's result is bit-identical
-// whatever the batch around it, whichever of the two runs, and with or without
-// the invalid indices written out.  The smallest calls, and many rows of few
-// heads and columns, run f32_row_kernel instead (f32_by_rows).
+// whichever of the two runs, and with or without the invalid indices written
+// out.  The smallest calls, and many rows of few heads and columns, run
+// f32_row_kernel instead (f32_by_rows: by the call's shape alone), which sums
+// in another order.
 //
 // What bounds it: at Q=8 H=16 Dc=512 Dp=64 S=1024 the call needs 24 MB
 // (5 us) and 0.29 GFLOP; it takes 19.5 us, two launches (16 + 4) of a few
